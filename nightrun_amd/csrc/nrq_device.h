@@ -690,64 +690,42 @@ __device__ __forceinline__ float wg_chain_nonneg(const float* __restrict__ a, in
   return s;
 }
 
-// musl scalbnf
-__device__ __forceinline__ float dev_scalbnf(float x, int n) {
-  float y = x;
-  if (n > 127) {
-    y *= __uint_as_float(0x7f000000u);
-    n -= 127;
-    if (n > 127) {
-      y *= __uint_as_float(0x7f000000u);
-      n -= 127;
-      if (n > 127) n = 127;
-    }
-  } else if (n < -126) {
-    y *= __uint_as_float(0x00800000u) * __uint_as_float(0x4b800000u);
-    n += 126 - 24;
-    if (n < -126) {
-      y *= __uint_as_float(0x00800000u) * __uint_as_float(0x4b800000u);
-      n += 126 - 24;
-      if (n < -126) n = -126;
-    }
-  }
-  return y * __uint_as_float((uint32_t)(0x7f + n) << 23);
-}
-
 // musl expf (FreeBSD e_expf.c algorithm): x = k ln2 + r, exp(r) from the
-// two-term Remez form, scaled by 2^k.
-__device__ inline float dev_expf(float x) {
+// two-term Remez form, scaled by 2^k (scalbnf: k past f32's exponents in two
+// exact-then-rounded steps). Every range of x runs the same instructions and
+// selects pick its result, so a wave of mixed arguments takes one pass, not
+// the sum of four branches. r*c / (2 - c) has its operands in [2^-27, 1/8] and
+// [1.6, 2.4], so the quotient needs no scaling: a reciprocal, one Newton step
+// and two residual corrections (Markstein) give the rounded value. Equal to
+// the branching form with the IEEE divide on all 2^32 arguments.
+__device__ __forceinline__ float dev_expf(float x) {
   const float ln2hi = 6.9314575195e-01f, ln2lo = 1.4286067653e-06f, invln2 = 1.4426950216e+00f;
   const float P1 = 1.6666625440e-1f, P2 = -2.7667332906e-3f;
-  uint32_t hx = __float_as_uint(x);
-  const int sign = (int)(hx >> 31);
-  hx &= 0x7fffffffu;
-  if (hx >= 0x42aeac50u) {
-    if (hx > 0x7f800000u) return x;
-    if (hx >= 0x42b17218u && !sign) return x * __uint_as_float(0x7f000000u);
-    if (sign && hx >= 0x42cff1b5u) return 0.0f;
-  }
-  int k;
-  float hi, lo;
-  if (hx > 0x3eb17218u) {
-    if (hx > 0x3f851592u)
-      k = (int)(invln2 * x + (sign ? -0.5f : 0.5f));
-    else
-      k = 1 - sign - sign;
-    const float kf = (float)k;
-    hi = x - kf * ln2hi;
-    lo = kf * ln2lo;
-    x = hi - lo;
-  } else if (hx > 0x39000000u) {
-    k = 0;
-    hi = x;
-    lo = 0.0f;
-  } else {
-    return 1.0f + x;
-  }
-  const float xx = x * x;
-  const float c = x - xx * (P1 + xx * P2);
-  const float y = 1.0f + (x * c / (2.0f - c) - lo + hi);
-  return k == 0 ? y : dev_scalbnf(y, k);
+  const uint32_t hx = __float_as_uint(x) & 0x7fffffffu;
+  const bool neg = (int)__float_as_uint(x) < 0;
+  int k = rust_f32_to_i32(invln2 * x + (neg ? -0.5f : 0.5f));
+  k = hx > 0x3f851592u ? k : (neg ? -1 : 1);
+  k = hx > 0x3eb17218u ? k : 0;
+  const float kf = (float)k;
+  const float hi = x - kf * ln2hi, lo = kf * ln2lo;
+  const float r = hi - lo;
+  const float rr = r * r;
+  const float c = r - rr * (P1 + rr * P2);
+  const float num = r * c, den = 2.0f - c;
+  float rc = __builtin_amdgcn_rcpf(den);
+  rc = fmaf(fmaf(-den, rc, 1.0f), rc, rc);
+  float q = num * rc;
+  q = fmaf(fmaf(-den, q, num), rc, q);
+  q = fmaf(fmaf(-den, q, num), rc, q);
+  const float y = 1.0f + (q - lo + hi);
+  // scalbnf(y, k) for the k that reach it, -150 .. 128
+  const float f1 = __uint_as_float(k > 127 ? 0x7f000000u : k < -126 ? 0x0c800000u : 0x3f800000u);
+  const int k2 = k > 127 ? k - 127 : k < -126 ? k + 102 : k;
+  float e = y * f1 * __uint_as_float((uint32_t)(0x7f + k2) << 23);
+  e = hx > 0x39000000u ? e : 1.0f + x;
+  e = neg && hx >= 0x42cff1b5u ? 0.0f : e;
+  e = !neg && hx >= 0x42b17218u ? x * __uint_as_float(0x7f000000u) : e;
+  return hx > 0x7f800000u ? x : e;
 }
 
 }  // namespace nrq
