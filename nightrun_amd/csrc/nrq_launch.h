@@ -118,6 +118,28 @@ int launch_quantize_q8k(const QuantLaunch& L);
 // Q4_K/Q6_K/Q8_0 per-(row, block) exact integer sums (test/diagnostic path).
 int launch_block_sums(int dtype, const void* w, const void* x, int32_t* out, int rows, int bpr, void* stream);
 
+// Prefill attention of `tokens` tokens at positions base.. (nrq_attn.hip),
+// head_dim 64 or 128. qt holds the roped queries in tiles of kPfRows rows,
+// [n_kv][tiles][head_dim][kPfRows], row (token, head of the group) =
+// token * gqa + head; scratch holds the attention weights of as many tiles as
+// fit. out and the optional quantized rows as in the other attention kernels.
+constexpr int kPfRows = 4;
+inline int pf_tiles(int tokens, int gqa) { return (tokens * gqa + kPfRows - 1) / kPfRows; }
+struct PfAttnLaunch {
+  const float* qt;
+  const uint16_t* kc;
+  const uint16_t* vc;
+  float* scratch;
+  size_t scratch_bytes;
+  float* out;
+  uint8_t* out_q8;
+  uint8_t* out_q8k;
+  int n_heads, n_kv, head_dim, ctx, layer, base, tokens;
+  float scale;
+  void* stream;
+};
+int launch_pf_attention(const PfAttnLaunch& L);
+
 // Sets the message nrq_last_error() returns on this thread (nrq_api.hip).
 void set_last_error(const char* msg);
 // The model frees `dev` (a hipMalloc'd buffer its tensors point into) when destroyed.

@@ -362,7 +362,8 @@ __global__ __launch_bounds__(256) void rope_append_kernel(float* __restrict__ q,
                                                           const int* __restrict__ ctl, int n_heads, int n_kv_heads,
                                                           int hd, int ctx, int layer, uint16_t* __restrict__ kc,
                                                           uint16_t* __restrict__ vc, const float* __restrict__ qn,
-                                                          const float* __restrict__ kn, float eps, int neox) {
+                                                          const float* __restrict__ kn, float eps, int neox,
+                                                          float* __restrict__ qt, int nrb) {
   __shared__ __align__(16) float raw[4][128];
   __shared__ __align__(16) float sqs[4][128];
   const int i = blockIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63, half = hd / 2;
@@ -390,6 +391,10 @@ __global__ __launch_bounds__(256) void rope_append_kernel(float* __restrict__ q,
   auto kvi = [&](int d) {
     return ((size_t)layer * n_kv_heads + hh) * hd * ctx + (size_t)(d >> 3) * ctx8 + (size_t)pos * 8 + (d & 7);
   };
+  // with qt, the query goes to row `row` of its KV head's tiles instead
+  const int gqa = n_heads / n_kv_heads, row = i * gqa + hh % gqa;
+  float* qd = qt ? qt + ((size_t)(hh / gqa) * nrb + row / kPfRows) * hd * kPfRows + row % kPfRows : qi;
+  const int qs = qt ? kPfRows : 1;
   for (int j = lane; j < half; j += 64) {
     const int ia = neox ? j : 2 * j, ib = neox ? j + half : 2 * j + 1;
     const float cs = cst[2 * j], sn = cst[2 * j + 1];
@@ -400,8 +405,8 @@ __global__ __launch_bounds__(256) void rope_append_kernel(float* __restrict__ q,
     }
     const float ra = a * cs - b * sn, rb = a * sn + b * cs;
     if (isq) {
-      qi[ia] = ra;
-      qi[ib] = rb;
+      qd[ia * qs] = ra;
+      qd[ib * qs] = rb;
     } else {
       kc[kvi(ia)] = (uint16_t)f32_to_f16_bits(ra);
       kc[kvi(ib)] = (uint16_t)f32_to_f16_bits(rb);
@@ -1478,6 +1483,8 @@ struct nrq_model {
   float *battn = nullptr, *bgate = nullptr, *bup = nullptr, *brope = nullptr;
   uint8_t *bxq = nullptr, *bxq2 = nullptr;
   int* btok = nullptr;
+  float *bqt = nullptr, *batt = nullptr;  // launch_pf_attention's query tiles and weights
+  size_t batt_bytes = 0;
   // Sampler (sample.rs:5-21): temperature <= 0 is greedy
   float samp_t = 0.0f, samp_p = 1.0f;
   unsigned long long* rng = nullptr;  // device word, seed | 1
@@ -1817,10 +1824,36 @@ AttGroupCfg att_group(const nrq_model_config& c) {
   return g;
 }
 
+// The tiled prefill attention (nrq_attn.hip) takes a chunk of B tokens of
+// 64- and 128-wide heads from 2048 (token, head) rows: below that its values
+// launch has too few waves for the chip (a wave owns four rows), and its three
+// launches cost more than one. Whole prefill of two layers, other kernels ->
+// tiles, us: Llama-3.2-1B widths, 32 tokens 313 -> 324 at position 0 and 541
+// -> 580 at 3000; 64 tokens 376 -> 374 and 804 -> 650; 512 tokens 1312 -> 993
+// and 4632 -> 1827. Qwen3-4B widths, 64 tokens 308 -> 312 and 726 -> 617; 512
+// tokens 1225 -> 987 and 4441 -> 2398. NRQ_ATT_TILES=0 / 1 forces the choice.
+bool att_tiles(const nrq_model* m, int B) {
+  const auto& c = m->cfg;
+  if (!m->batt || (c.head_dim != 64 && c.head_dim != 128)) return false;
+  const char* env = getenv("NRQ_ATT_TILES");
+  if (env && (env[0] == '0' || env[0] == '1')) return env[0] == '1';
+  return (long long)B * c.n_heads >= 2048;
+}
+
+// Attention weights of one pass of the tiled attention: a 512-token chunk of 32
+// heads up to position 4096, more passes beyond. NRQ_ATT_SCRATCH (bytes) sets
+// another limit.
+constexpr size_t kPfScratch = (size_t)256 << 20;
+
 int prefill_alloc(nrq_model* m) {
   if (m->bx) return NRQ_OK;
   const auto& c = m->cfg;
   const size_t B = kMaxBatch, maxd = (size_t)m->maxd;
+  // at most a chunk's rows over the whole context; at least one tile per KV head
+  const size_t tile = (size_t)c.n_kv_heads * ((c.ctx + 63) & ~63) * nrq::kPfRows * 4;
+  const size_t tiles = nrq::pf_tiles(std::min(kMaxBatch, c.ctx), c.n_heads / c.n_kv_heads);
+  const char* env = getenv("NRQ_ATT_SCRATCH");
+  m->batt_bytes = std::max(tile, std::min(tile * tiles, env ? (size_t)strtoull(env, nullptr, 10) : kPfScratch));
   struct {
     void** p;
     size_t bytes;
@@ -1831,9 +1864,15 @@ int prefill_alloc(nrq_model* m) {
       {(void**)&m->battn, B * m->att_dim * 4},  {(void**)&m->bgate, B * c.ffn_dim * 4},
       {(void**)&m->bup, B * c.ffn_dim * 4},     {(void**)&m->brope, B * c.head_dim * 4},
       {(void**)&m->bxq, B * act_bytes(NRQ_Q8_0, maxd) + 64}, {(void**)&m->bxq2, B * act_bytes(NRQ_Q4_K, maxd) + 64},
+      {(void**)&m->bqt, (B * m->att_dim + (size_t)c.n_kv_heads * nrq::kPfRows * c.head_dim) * 4},
       {(void**)&m->btok, B * 4},
   };
   for (auto& a : allocs) MHIP(hipMalloc(a.p, a.bytes));
+  // without room for the weights the other attention kernels take every chunk
+  if (hipMalloc((void**)&m->batt, m->batt_bytes) != hipSuccess) {
+    m->batt = nullptr;
+    (void)hipGetLastError();
+  }
   return NRQ_OK;
 }
 
@@ -1945,6 +1984,8 @@ int enqueue_prefill(nrq_model* m, int B) {
   if (hipGetLastError() != hipSuccess) return mfail(NRQ_ERR_DEVICE, "model: embed launch failed");
   const float scale = m->att_scale;
   const float* pending = nullptr;
+  const bool tiles = att_tiles(m, B);
+  const int gqa = c.n_heads / c.n_kv_heads;
   int rc;
   for (int l = 0; l < c.n_layers; l++) {
     const Layer& Ly = m->L[l];
@@ -1961,15 +2002,20 @@ int enqueue_prefill(nrq_model* m, int B) {
     hipLaunchKernelGGL(nrq::rope_append_kernel, dim3(B, (c.n_heads + c.n_kv_heads + 3) / 4), dim3(256), 0, m->stream,
                        m->bq, m->bk, m->bv, m->brope,
                        m->ctl, c.n_heads, c.n_kv_heads, c.head_dim, c.ctx, l, m->kc, m->vc, Ly.q_norm, Ly.k_norm,
-                       c.norm_eps, m->rope_neox);
+                       c.norm_eps, m->rope_neox, tiles ? m->bqt : nullptr, nrq::pf_tiles(B, gqa));
     if (hipGetLastError() != hipSuccess) return mfail(NRQ_ERR_DEVICE, "model: rope launch failed");
     {
       const bool q8 = Ly.m[3].dt == NRQ_Q8_0;
       const AttGroupCfg gk = att_group(c);
       // a K-quant o projection's Q8_K input, written by the attention when a
       // workgroup's heads are one 256-value block
-      const bool q8k = !q8 && gk.fn && gk.gh * c.head_dim == 256;
-      if (gk.fn) {
+      const bool q8k = !q8 && (tiles ? gqa * c.head_dim % 256 == 0 : gk.fn && gk.gh * c.head_dim == 256);
+      if (tiles) {
+        const nrq::PfAttnLaunch P{m->bqt, m->kc, m->vc, m->batt, m->batt_bytes, m->battn, q8 ? m->bxq : nullptr,
+                                  q8k ? m->bxq2 : nullptr, c.n_heads, c.n_kv_heads, c.head_dim, c.ctx, l, m->host_pos,
+                                  B, scale, m->stream};
+        if (nrq::launch_pf_attention(P)) return mfail(NRQ_ERR_DEVICE, "model: attention launch failed");
+      } else if (gk.fn) {
         hipLaunchKernelGGL(gk.fn, dim3(c.n_heads / gk.gh, B), dim3(gk.nt), gk.lds, m->stream, m->bq, m->ctl, c.n_heads,
                            c.n_kv_heads, c.ctx, l, scale, m->kc, m->vc, m->battn, q8 ? m->bxq : nullptr,
                            q8k ? m->bxq2 : nullptr);
@@ -2472,7 +2518,7 @@ int nrq_model_destroy(nrq_model* m) {
   if (m->graph) hipGraphDestroy(m->graph);
   void* bufs[] = {m->freqs, m->rope_cs, m->kc, m->vc, m->x, m->x2, m->xb, m->q, m->k, m->v, m->attn, m->gate, m->up, m->xb2,
                   m->logits, m->xq, m->xq2, m->ctl, m->out_tokens, m->owned, m->bx, m->bxb, m->bxn, m->bq,
-                  m->bk, m->bv, m->battn, m->bgate, m->bup, m->brope, m->bxq, m->bxq2, m->btok, m->rng, m->samp_part};
+                  m->bk, m->bv, m->battn, m->bgate, m->bup, m->brope, m->bxq, m->bxq2, m->btok, m->bqt, m->batt, m->rng, m->samp_part};
   for (void* p : bufs)
     if (p) hipFree(p);
   if (m->stream) hipStreamDestroy(m->stream);

@@ -544,3 +544,37 @@ def test_kquant_embedding_matches_oracle(gpu, oracle, edt):
     prompt = np.random.default_rng(edt).integers(0, TINY["vocab"], 30).astype(np.uint32)
     run_pair(oracle, TINY, w, 64, prompt, 6)
     run_pair(oracle, TINY, w, 64, prompt, 6, prefill=True)
+
+
+# ---- the tiled prefill attention (NRQ_ATT_TILES=1 takes it below its default size) ----------
+
+TILES_GQA3 = dict(TINY, dim=256, n_heads=12, n_kv_heads=4)  # tiles of rows of two tokens; no 256-wide o block per group
+TILES = {"gqa2-hd64": TINY, "gqa3-hd64": TILES_GQA3, "gqa4-hd64": TINY_GQA4, "gqa2-hd128": QWEN_HD128,
+         "gqa1-hd64": dict(TINY, n_kv_heads=4)}
+
+
+@pytest.mark.parametrize("fmt", ["q8_0", "q4k_m"])
+@pytest.mark.parametrize("cfg,n,scratch", [("gqa2-hd64", 1, None), ("gqa3-hd64", 67, None), ("gqa3-hd64", 257, "1"),
+                                           ("gqa4-hd64", 513, None), ("gqa4-hd64", 300, "200000"),
+                                           ("gqa2-hd128", 290, None), ("gqa2-hd128", 33, "1"),
+                                           ("gqa1-hd64", 130, None)])
+def test_prefill_attention_tiles(gpu, oracle, monkeypatch, cfg, n, scratch, fmt):
+    """The three-launch prefill attention at the edges of its tiles: row counts that
+    do not fill the last four-row tile, positions across the 64-, 256- and
+    32-position steps, a chunk at position 512, and a weights scratch that holds
+    a few tiles (NRQ_ATT_SCRATCH; at least one per KV head), so that one chunk
+    takes several passes. Q8_0 and Q8_K output rows; bit-exact."""
+    monkeypatch.setenv("NRQ_ATT_TILES", "1")
+    if scratch:
+        monkeypatch.setenv("NRQ_ATT_SCRATCH", scratch)
+    c = TILES[cfg]
+    w = oracle.gen_model(c, 900 + n, qk_norm="recipe" in c)
+    if fmt == "q4k_m":
+        shapes = oracle.layer_shapes(c)
+        for l, lw in enumerate(w["layers"]):
+            for i, name in enumerate(oracle.LAYER_MATS):
+                rows, cols = shapes[name]
+                lw[name] = oracle.gen_weights(Q4K_M[name], 5500 + 16 * l + i, rows, cols)
+                lw["dtypes"][name] = Q4K_M[name]
+    prompt = np.random.default_rng(n).integers(0, c["vocab"], n).astype(np.uint32)
+    run_pair(oracle, c, w, n + 40, prompt, 3, prefill=True)
