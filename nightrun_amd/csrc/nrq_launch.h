@@ -103,6 +103,10 @@ struct MatmulGroupLaunch {
   void* stream;
 };
 int launch_mmt_group(int dtype, const MatmulGroupLaunch& G);
+// Q8_0 matrices at 64 tokens and more (nrq_mm8.hip); mm8_fits: the kernel takes
+// the shape and is the faster one (any_size: only the former).
+bool mm8_fits(const MatmulGroupLaunch& G, bool any_size);
+int launch_mm8(const MatmulGroupLaunch& G);
 // Two such groups, of two different K-quant formats over one activation (q|k
 // Q4_K and v Q6_K), in one launch; NRQ_LAUNCH_BAD_ARG when the kernel does not
 // take the pair.

@@ -634,6 +634,50 @@ def test_matmul_q8_0_spans(gpu, oracle, monkeypatch):
                            f"spans forced {forced} rows {rows} cols {cols} batch {batch}")
 
 
+@pytest.mark.parametrize("rows_list,bpr,batch", [((64,), 8, 64), ((100,), 10, 65), ((6144, 128), 8, 95),
+                                                 ((130, 64, 7000), 12, 129), ((8200, 8300), 10, 260),
+                                                 ((3000, 40, 3200), 34, 67), ((1531,), 9, 300),
+                                                 ((8200, 8300), 11, 260), ((64,), 31, 64)])
+def test_matmul_q8_0_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch):
+    """The Q8_0 kernel of 64 tokens and more (one or two 32 x 32 tiles per wave, stages of
+    8 blocks whose last one starts early, as the last row and token tiles do): the smallest
+    tile, short last tiles and stages, groups with one short matrix, odd block counts
+    (rows two bytes past a dword), and weight scales that are negative, zero, subnormal, the largest f16
+    and, in the last matrix, infinite and NaN, against quants of -128."""
+    import torch
+
+    from nightrun_amd import device
+
+    if rows_list == (64,):
+        monkeypatch.setenv("NRQ_MMT_NB", "8")
+        monkeypatch.setenv("NRQ_MMT_SPLITS", "1")
+    cols = 32 * bpr
+    xs = oracle.quantize_act(1, oracle.Rng(940 + bpr).normal(batch * cols))
+    rng = np.random.default_rng(bpr)
+    ws = []
+    for i, r in enumerate(rows_list):
+        w = np.ascontiguousarray(oracle.gen_weights(1, 950 + i + bpr, r, cols)).view(np.uint8).reshape(-1, 34).copy()
+        special = [0x8000, 0x0001, 0x83FF, 0x7BFF, 0xBC00, 0x0000]
+        if i == len(rows_list) - 1:
+            special += [0x7C00, 0xFC00, 0x7E00]
+        at = rng.integers(0, len(w), 60)
+        w[at, :2] = np.resize(np.array(special, np.uint16), 60).view(np.uint8).reshape(-1, 2)
+        w[rng.integers(0, len(w), 40), 2:] = 0x80
+        ws.append(w.reshape(-1))
+    ys = [torch.empty(batch * r, dtype=torch.float32, device="cuda") for r in rows_list]
+    # the activation 4 bytes past an aligned address
+    buf = torch.zeros(4 + xs.nbytes, dtype=torch.uint8, device="cuda")
+    buf[4:] = torch.from_numpy(np.ascontiguousarray(xs).view(np.uint8).reshape(-1)).cuda()
+    device.matmul_group(1, ys, [torch.from_numpy(w).cuda() for w in ws], list(rows_list), buf[4:], cols, batch)
+    torch.cuda.synchronize()
+    for i, r in enumerate(rows_list):
+        want = oracle.matmul(1, 0, ws[i], xs, r, cols, batch, threads=THREADS)
+        got = ys[i].cpu().numpy()
+        nan = np.isnan(want)
+        assert np.array_equal(np.isnan(got), nan)
+        assert_bitwise(got[~nan], want[~nan], f"matrix {i} rows {r} bpr {bpr} batch {batch}")
+
+
 @pytest.mark.parametrize("dtype", [1, 2, 3])
 def test_matmul_group(gpu, oracle, dtype):
     """nrq_dev_matmul_group (Acts::matmul_group, infer.rs:180-228): every
