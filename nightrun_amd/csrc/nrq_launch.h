@@ -107,6 +107,9 @@ int launch_mmt_group(int dtype, const MatmulGroupLaunch& G);
 // the shape and is the faster one (any_size: only the former).
 bool mm8_fits(const MatmulGroupLaunch& G, bool any_size);
 int launch_mm8(const MatmulGroupLaunch& G);
+// Q4_K matrices at 64 tokens and more (nrq_mmk.hip), as for nrq_mm8.hip
+bool mmk_fits(const MatmulGroupLaunch& G, bool any_size);
+int launch_mmk(const MatmulGroupLaunch& G);
 // Two such groups, of two different K-quant formats over one activation (q|k
 // Q4_K and v Q6_K), in one launch; NRQ_LAUNCH_BAD_ARG when the kernel does not
 // take the pair.

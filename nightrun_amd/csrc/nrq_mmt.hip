@@ -787,16 +787,19 @@ int md2_launch_ks(const MatmulGroupLaunch& G0, const MatmulGroupLaunch& G1, int 
   return md2_launch_t<F0, F1, 2>(G0, G1);
 }
 
-// Q8_0 on the kernel of nrq_mm8.hip, unless a tuning override names another.
-bool md_takes_mm8(const MatmulGroupLaunch& G) {
+// Q8_0 on the kernel of nrq_mm8.hip, Q4_K on that of nrq_mmk.hip, unless a tuning
+// override names another (8 buffers in 1 split: these).
+bool md_takes(const MatmulGroupLaunch& G, bool (*fits)(const MatmulGroupLaunch&, bool)) {
   const char *nb = getenv("NRQ_MMT_NB"), *ks = getenv("NRQ_MMT_SPLITS"), *db = getenv("NRQ_MMT_DB");
   const bool forced = nb && atoi(nb) == 8 && ks && atoi(ks) == 1;
   if (!forced && ((nb && nb[0]) || (ks && ks[0]) || (db && db[0]))) return false;
-  return mm8_fits(G, forced);
+  return fits(G, forced);
 }
+bool md_takes_mm8(const MatmulGroupLaunch& G) { return md_takes(G, mm8_fits); }
 
 int md_group(int dtype, const MatmulGroupLaunch& G) {
   if (dtype == kQ8_0 && md_takes_mm8(G)) return launch_mm8(G);
+  if (dtype == kQ4K && md_takes(G, mmk_fits)) return launch_mmk(G);
   long row_tiles = 0;
   for (int i = 0; i < G.nmat; i++) row_tiles += (G.rows[i] + 31) / 32;
   const int ks = md_choose(dtype, row_tiles, G.batch, G.bpr);
@@ -811,7 +814,7 @@ int md_group(int dtype, const MatmulGroupLaunch& G) {
 // on two, which spill). Q8_0: one (on the Llama-3.2-1B shapes at M = 64 one
 // buffer beat two and a ring of four by 4-20%).
 int md_buffers(int dtype, int ks, int batch, int bpr) {
-  const char* nb = getenv("NRQ_MMT_NB");  // tuning override: 1, 2 or 4 (4: Q8_0 only); 8: nrq_mm8.hip, see md_takes_mm8
+  const char* nb = getenv("NRQ_MMT_NB");  // tuning override: 1, 2 or 4 (4: Q8_0 only); 8: see md_takes
   if (nb && nb[0]) return atoi(nb);
   const char* env = getenv("NRQ_MMT_DB");  // tuning override: 0 (one buffer) or 1 (two)
   if (env && env[0]) return env[0] == '1' ? 2 : 1;

@@ -678,6 +678,47 @@ def test_matmul_q8_0_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch
         assert_bitwise(got[~nan], want[~nan], f"matrix {i} rows {r} bpr {bpr} batch {batch}")
 
 
+@pytest.mark.parametrize("rows_list,bpr,batch,forced", [((128,), 1, 64, True), ((200,), 3, 65, True),
+                                                        ((130, 300, 128), 2, 95, True), ((5000, 4700), 2, 130, False),
+                                                        ((9000, 8200), 5, 460, False)])
+def test_matmul_q4k_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch, forced):
+    """The Q4_K kernel of 64 tokens and more (one or two tiles of 32 tokens per wave): the
+    smallest tile, short last tiles, one block and several, and in every matrix blocks of
+    the largest scales, mins and quants against activations of -128 and 127 (their sums
+    pass 2^24, where the f32 steps round), zero scales and the f16 extremes of d."""
+    import torch
+
+    from nightrun_amd import device
+
+    if forced:
+        monkeypatch.setenv("NRQ_MMT_NB", "8")
+        monkeypatch.setenv("NRQ_MMT_SPLITS", "1")
+    cols = 256 * bpr
+    rng = np.random.default_rng(17 * bpr + batch)
+    xs = np.ascontiguousarray(oracle.quantize_act(2, oracle.Rng(960 + bpr).normal(batch * cols))).view(np.uint8)
+    xs = xs.reshape(-1, 292).copy()
+    for k, v in enumerate((-128, 127, -128)):  # whole blocks, bsums with them
+        at = rng.integers(0, len(xs), 8)
+        xs[at, 4:260] = np.int8(v).view(np.uint8)
+        xs[at, 260:] = np.full(16, 16 * v, np.int16).view(np.uint8)
+    ws = []
+    for i, r in enumerate(rows_list):
+        w = np.ascontiguousarray(oracle.gen_weights(2, 970 + i + bpr, r, cols)).view(np.uint8).reshape(-1, 144).copy()
+        at = rng.integers(0, len(w), 40)
+        w[at, 4:] = 0xFF  # scales and mins 63, quants 15
+        w[rng.integers(0, len(w), 10), 4:16] = 0
+        at = rng.integers(0, len(w), 12)
+        w[at, :4] = np.resize(np.array([0x8001, 0x7BFF, 0xBC00, 0x0000], np.uint16), 24).view(np.uint8).reshape(-1, 4)
+        ws.append(w.reshape(-1))
+    ys = [torch.empty(batch * r, dtype=torch.float32, device="cuda") for r in rows_list]
+    device.matmul_group(2, ys, [torch.from_numpy(w).cuda() for w in ws], list(rows_list),
+                        torch.from_numpy(xs.reshape(-1)).cuda(), cols, batch)
+    torch.cuda.synchronize()
+    for i, r in enumerate(rows_list):
+        want = oracle.matmul(2, 0, ws[i], xs.reshape(-1), r, cols, batch, threads=THREADS)
+        assert_bitwise(ys[i].cpu().numpy(), want, f"matrix {i} rows {r} bpr {bpr} batch {batch}")
+
+
 @pytest.mark.parametrize("dtype", [1, 2, 3])
 def test_matmul_group(gpu, oracle, dtype):
     """nrq_dev_matmul_group (Acts::matmul_group, infer.rs:180-228): every
