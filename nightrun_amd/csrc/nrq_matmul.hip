@@ -1,10 +1,10 @@
 // Batched matmul (prefill): y[b][r] = dot(W[r,:], xs[b]).
 // The reference guarantees matmul == per-token matvec bit for bit
 // (kernels.rs:84-90, kquant.rs:566-569). Scalar order runs the int8-MFMA tile
-// kernels (nrq_mmt.hip, nrq_mmq.hip). AVX2 order runs the int8-MFMA tiles of
-// nrq_mma.hip from two tokens, and the decode kernel for one: both equal the
-// 1-wide AVX2 dot per token, as the reference's 4-wide tiles do
-// (kernels.rs:222-223).
+// kernels (nrq_mmt.hip, nrq_mmq.hip; from 64 tokens nrq_mm8.hip and
+// nrq_mmk.hip). AVX2 order runs the int8-MFMA tiles of nrq_mma.hip from two
+// tokens, and the decode kernel for one: both equal the 1-wide AVX2 dot per
+// token, as the reference's 4-wide tiles do (kernels.rs:222-223).
 #include "nrq_device.h"
 #include "nrq_launch.h"
 

@@ -322,7 +322,7 @@ long mmk_tiles(const MatmulGroupLaunch& G, int tok) {
 bool mmk_fits(const MatmulGroupLaunch& G, bool any_size) {
   for (int i = 0; i < G.nmat; i++)
     if (G.rows[i] < kRowsWg) return false;
-  return G.batch >= 64 && G.bpr <= (1 << 18) && (any_size || (G.bpr < 32 && mmk_tiles(G, 32) >= 300));
+  return G.batch >= 64 && G.bpr <= (1 << 17) && (any_size || (G.bpr < 32 && mmk_tiles(G, 32) >= 300));
 }
 
 int launch_mmk(const MatmulGroupLaunch& G) {
