@@ -41,7 +41,7 @@ struct QuantLaunch {
   void* dst;         // device blocks
   long long n;       // elements (multiple of the block size)
   void* stream;
-  const float* up = nullptr;  // Q8_K only: quantize swiglu(src, up), written back over src
+  const float* up = nullptr;  // Q8_K only: quantize swiglu(src, up)
 };
 
 // Scalar order: the streaming kernel (nrq_wstream.hip); AVX2 order: the

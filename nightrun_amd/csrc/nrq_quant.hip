@@ -39,19 +39,16 @@ __global__ __launch_bounds__(256) void quantize_q8_0_kernel(const float* __restr
 }
 
 // One Q8_K block per 256-thread workgroup: thread t loads value t (and with
-// `up` forms swiglu(src, up) = src / (1 + expf(-src)) * up, vec.rs:45-52,
-// written back over src), then the first half-wave quantizes the block,
+// `up` forms swiglu(src, up) = src / (1 + expf(-src)) * up, vec.rs:45-52, of
+// which only the blocks are kept), then the first half-wave quantizes the block,
 // lane r holding values 8r .. 8r+7 (q8k_half_lanes, nrq_device.h).
-__global__ __launch_bounds__(256) void quantize_q8k_kernel(float* __restrict__ src, uint8_t* __restrict__ dst,
+__global__ __launch_bounds__(256) void quantize_q8k_kernel(const float* __restrict__ src, uint8_t* __restrict__ dst,
                                                            const float* __restrict__ up) {
   __shared__ __align__(16) float s_v[256];
   const long long b = blockIdx.x;
   const int t = threadIdx.x;
   float v = src[b * 256 + t];
-  if (up) {
-    v = v / (1.0f + dev_expf(-v)) * up[b * 256 + t];
-    src[b * 256 + t] = v;
-  }
+  if (up) v = v / (1.0f + dev_expf(-v)) * up[b * 256 + t];
   s_v[t] = v;
   __syncthreads();
   if (t < 32) {
@@ -116,7 +113,7 @@ int launch_quantize_q8k(const QuantLaunch& L) {
   if (L.n % 256) return NRQ_LAUNCH_BAD_ARG;
   const long long nb = L.n / 256;
   hipLaunchKernelGGL(quantize_q8k_kernel, dim3((unsigned)nb), dim3(256), 0, (hipStream_t)L.stream,
-                     const_cast<float*>(L.src), (uint8_t*)L.dst, L.up);
+                     L.src, (uint8_t*)L.dst, L.up);
   return hipGetLastError() == hipSuccess ? 0 : NRQ_LAUNCH_FAILED;
 }
 
