@@ -85,9 +85,8 @@ int launch_matmul(int dtype, int order, const MatmulLaunch& L);
 // Scalar-order batched matmul on int8 MFMA: the 32 x 32 tiles of nrq_mmt.hip,
 // or for Q8_0 below 1024 rows the 16 x 16 tiles of nrq_mmq.hip.
 int launch_mmq(int dtype, const MatmulLaunch& L);
-// Prefill on 32-row x 32-token wave tiles (nrq_mmt.hip); mmt_fits: the kernel
-// handles the format and shape.
-bool mmt_fits(int dtype, const MatmulLaunch& L);
+// Prefill on 32-row x 32-token wave tiles (nrq_mmt.hip); NRQ_LAUNCH_BAD_ARG when
+// the kernel does not take the format and shape.
 int launch_mmt(int dtype, const MatmulLaunch& L);
 // Up to three matrices of one format and width sharing one activation (q|k|v,
 // gate|up) in one launch of the same kernel, y[i] = [batch][rows[i]].

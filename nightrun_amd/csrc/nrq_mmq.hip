@@ -138,8 +138,8 @@ int launch_mmq(int dtype, const MatmulLaunch& L) {
   hipStream_t st = (hipStream_t)L.stream;
   const uint8_t* w = (const uint8_t*)L.w;
   const uint8_t* x = (const uint8_t*)L.xs;
-  if (mmt_fits(dtype, L)) return launch_mmt(dtype, L);  // every Q4_K / Q6_K shape
-  if (dtype != kQ8_0) return NRQ_LAUNCH_BAD_ARG;
+  const int rc = launch_mmt(dtype, L);  // every Q4_K / Q6_K shape
+  if (rc != NRQ_LAUNCH_BAD_ARG || dtype != kQ8_0) return rc;
   hipLaunchKernelGGL(mmq_kernel<kQ8_0>, grid, dim3(256), 0, st, w, x, L.y, L.rows, L.bpr, L.batch, ntt, nrt);
   return hipGetLastError() == hipSuccess ? 0 : NRQ_LAUNCH_FAILED;
 }

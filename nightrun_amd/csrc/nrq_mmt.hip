@@ -43,6 +43,8 @@
 
 #include <stdio.h>
 #include <stdlib.h>
+#include <string.h>
+#include <unistd.h>
 
 namespace nrq {
 
@@ -692,7 +694,7 @@ MdMats md_mats(const MatmulGroupLaunch& G, int* nrt) {
 }
 
 template <int FMT, int KS, int NB>
-int md_launch_t(const MatmulGroupLaunch& G) {
+int md_launch_t(const MatmulGroupLaunch& G, int early_x) {
   int nrt = 0;
   const MdMats M = md_mats(G, &nrt);
   const int ntt = (G.batch + 31) / 32;
@@ -701,33 +703,54 @@ int md_launch_t(const MatmulGroupLaunch& G) {
   if (nwg > 0x7fffffffL) return NRQ_LAUNCH_BAD_ARG;
   const size_t lds = (size_t)KS * kMdScalDw * 4 + (KS > 1 ? (size_t)2 * KS * 1024 * 4 : 0) +
                      (FMT == kQ8_0 ? 0 : (size_t)KS * kMdStage);
-  // one buffer: the next block's activation windows load as soon as the
-  // current block's are staged (Q6_K, and Q4_K rows of 16+ blocks: down 30.5 ->
-  // 27.7 us, o 13.4 -> 12.4 us on the Qwen3-4B layer at M = 64; q|k|v, 10
-  // blocks, 13.4 -> 13.8 us, so not there), else with its weights
-  const char* ex = getenv("NRQ_MMT_EARLY_X");
-  const int early_x = ex && ex[0] ? ex[0] == '1' : (FMT == kQ6K || (FMT == kQ4K && G.bpr >= 16));
   hipLaunchKernelGGL((mmd_kernel<FMT, KS, NB>), dim3((unsigned)nwg), dim3(64 * KS), lds, (hipStream_t)G.stream, M,
                      (const uint8_t*)G.xs, G.bpr, G.batch, ntt, nrt, early_x);
   return hipGetLastError() == hipSuccess ? 0 : NRQ_LAUNCH_FAILED;
 }
 
 template <int FMT, int NB>
-int md_launch_ks(const MatmulGroupLaunch& L, int ks) {
-  if (ks >= 8) return md_launch_t<FMT, 8, NB>(L);
-  if (ks == 4) return md_launch_t<FMT, 4, NB>(L);
-  if (ks == 2) return md_launch_t<FMT, 2, NB>(L);
-  return md_launch_t<FMT, 1, NB>(L);
+int md_launch_ks(const MatmulGroupLaunch& L, int ks, int early_x) {
+  if (ks >= 8) return md_launch_t<FMT, 8, NB>(L, early_x);
+  if (ks == 4) return md_launch_t<FMT, 4, NB>(L, early_x);
+  if (ks == 2) return md_launch_t<FMT, 2, NB>(L, early_x);
+  return md_launch_t<FMT, 1, NB>(L, early_x);
 }
 
 // K-quant blocks (256 values) need one or two buffers; Q8_0 blocks (32
 // values) take a ring of four to keep enough loads in flight.
 template <int FMT>
-int md_launch(const MatmulGroupLaunch& L, int ks, int nb) {
+int md_launch(const MatmulGroupLaunch& L, int ks, int nb, int early_x) {
   if constexpr (FMT == kQ8_0) {
-    if (nb == 4) return md_launch_ks<FMT, 4>(L, ks);
+    if (nb == 4) return md_launch_ks<FMT, 4>(L, ks, early_x);
   }
-  return nb == 2 ? md_launch_ks<FMT, 2>(L, ks) : md_launch_ks<FMT, 1>(L, ks);
+  return nb == 2 ? md_launch_ks<FMT, 2>(L, ks, early_x) : md_launch_ks<FMT, 1>(L, ks, early_x);
+}
+
+// Tuning overrides, null where not set or empty: NRQ_MMT_SPLITS 1, 2, 4 or 8 splits;
+// NRQ_MMT_NB 1, 2 or 4 register buffers (4: Q8_0 only; 8 with one split: see md_takes);
+// NRQ_MMT_DB 0 (one buffer) or 1 (two); NRQ_MMT_EARLY_X 0 or 1. One pass over the
+// environment for all four, once per launch: the host bounds a launch of small
+// matrices, where lookups cost 5% (Q8_0 600 + 600 + 512 x 1024 at 8 tokens: 19
+// lookups, one set per matrix, 9.5 us; 4, 9.2; this 8.9. Q4_K 1139 x 1536 at 110:
+// 7.8 -> 7.5; Q8_0 700 x 1024 at 8, which reads none of them: 7.3 -> 6.9 with the
+// shape tested first).
+struct MdTune {
+  const char *splits = nullptr, *nb = nullptr, *db = nullptr, *early_x = nullptr;
+};
+MdTune md_tune() {
+  MdTune t;
+  const struct {
+    const char* name;
+    const char** to;
+  } vars[] = {{"SPLITS=", &t.splits}, {"NB=", &t.nb}, {"DB=", &t.db}, {"EARLY_X=", &t.early_x}};
+  for (char** e = environ; e && *e; e++) {
+    if (**e != 'N' || strncmp(*e, "NRQ_MMT_", 8)) continue;
+    for (const auto& v : vars) {
+      const size_t n = strlen(v.name);
+      if (!*v.to && !strncmp(*e + 8, v.name, n) && (*e)[8 + n]) *v.to = *e + 8 + n;
+    }
+  }
+  return t;
 }
 
 // Block splits per tile: none when the tiles alone give four waves per CU
@@ -738,10 +761,9 @@ int md_launch(const MatmulGroupLaunch& L, int ks, int nb) {
 // or two blocks; the o projection's 16-block rows take 8 with the early
 // activation loads, 12.4 -> 12.0 us). Measured on the Qwen3-4B layer shapes
 // at M = 64 and M = 512.
-int md_choose(int dtype, long row_tiles, int batch, int bpr) {
-  const char* env = getenv("NRQ_MMT_SPLITS");  // tuning override: 1, 2, 4 or 8
-  if (env && env[0]) {
-    const int ks = atoi(env);
+int md_choose(const MdTune& T, int dtype, long row_tiles, int batch, int bpr) {
+  if (T.splits) {
+    const int ks = atoi(T.splits);
     if (ks == 1 || ks == 2 || ks == 4 || ks == 8) return ks;
   }
   const long tiles = row_tiles * ((batch + 31) / 32);
@@ -758,16 +780,19 @@ int md_choose(int dtype, long row_tiles, int batch, int bpr) {
   return ks;
 }
 
-int md_buffers(int dtype, int ks, int batch, int bpr);
+int md_buffers(const MdTune& T, int dtype, int ks, int batch, int bpr);
 
-// the early activation loads of md_launch_t, by format and row length
-int md_early_x(int fmt, int bpr) {
-  const char* ex = getenv("NRQ_MMT_EARLY_X");
-  return ex && ex[0] ? ex[0] == '1' : (fmt == kQ6K || (fmt == kQ4K && bpr >= 16));
+// The early activation loads of mmd_kernel, by format and row length. With
+// one buffer the next block's activation windows load as soon as the
+// current block's are staged (Q6_K, and Q4_K rows of 16+ blocks: down 30.5 ->
+// 27.7 us, o 13.4 -> 12.4 us on the Qwen3-4B layer at M = 64; q|k|v, 10
+// blocks, 13.4 -> 13.8 us, so not there), else with its weights
+int md_early_x(const MdTune& T, int fmt, int bpr) {
+  return T.early_x ? T.early_x[0] == '1' : (fmt == kQ6K || (fmt == kQ4K && bpr >= 16));
 }
 
 template <int F0, int F1, int KS>
-int md2_launch_t(const MatmulGroupLaunch& G0, const MatmulGroupLaunch& G1) {
+int md2_launch_t(const MdTune& T, const MatmulGroupLaunch& G0, const MatmulGroupLaunch& G1) {
   int nrt0 = 0, nrt1 = 0;
   const MdMats M0 = md_mats(G0, &nrt0), M1 = md_mats(G1, &nrt1);
   const int ntt = (G0.batch + 31) / 32;
@@ -776,36 +801,35 @@ int md2_launch_t(const MatmulGroupLaunch& G0, const MatmulGroupLaunch& G1) {
   const size_t lds = (size_t)KS * kMdScalDw * 4 + (size_t)2 * KS * 1024 * 4 + (size_t)KS * kMdStage;
   hipLaunchKernelGGL((mmd2_kernel<F0, F1, KS>), dim3((unsigned)(nwg0 + nwg1)), dim3(64 * KS), lds,
                      (hipStream_t)G0.stream, M0, M1, (const uint8_t*)G0.xs, G0.bpr, G0.batch, ntt, nrt0, nrt1,
-                     (int)nwg0, md_early_x(F0, G0.bpr), md_early_x(F1, G1.bpr));
+                     (int)nwg0, md_early_x(T, F0, G0.bpr), md_early_x(T, F1, G1.bpr));
   return hipGetLastError() == hipSuccess ? 0 : NRQ_LAUNCH_FAILED;
 }
 
 template <int F0, int F1>
-int md2_launch_ks(const MatmulGroupLaunch& G0, const MatmulGroupLaunch& G1, int ks) {
-  if (ks >= 8) return md2_launch_t<F0, F1, 8>(G0, G1);
-  if (ks == 4) return md2_launch_t<F0, F1, 4>(G0, G1);
-  return md2_launch_t<F0, F1, 2>(G0, G1);
+int md2_launch_ks(const MdTune& T, const MatmulGroupLaunch& G0, const MatmulGroupLaunch& G1, int ks) {
+  if (ks >= 8) return md2_launch_t<F0, F1, 8>(T, G0, G1);
+  if (ks == 4) return md2_launch_t<F0, F1, 4>(T, G0, G1);
+  return md2_launch_t<F0, F1, 2>(T, G0, G1);
 }
 
 // Q8_0 on the kernel of nrq_mm8.hip, Q4_K on that of nrq_mmk.hip, unless a tuning
 // override names another (8 buffers in 1 split: these).
-bool md_takes(const MatmulGroupLaunch& G, bool (*fits)(const MatmulGroupLaunch&, bool)) {
-  const char *nb = getenv("NRQ_MMT_NB"), *ks = getenv("NRQ_MMT_SPLITS"), *db = getenv("NRQ_MMT_DB");
-  const bool forced = nb && atoi(nb) == 8 && ks && atoi(ks) == 1;
-  if (!forced && ((nb && nb[0]) || (ks && ks[0]) || (db && db[0]))) return false;
-  return fits(G, forced);
+bool md_takes(const MdTune& T, int dtype, const MatmulGroupLaunch& G) {
+  if (dtype != kQ8_0 && dtype != kQ4K) return false;
+  const bool forced = T.nb && atoi(T.nb) == 8 && T.splits && atoi(T.splits) == 1;
+  if (!forced && (T.nb || T.splits || T.db)) return false;
+  return dtype == kQ8_0 ? mm8_fits(G, forced) : mmk_fits(G, forced);
 }
-bool md_takes_mm8(const MatmulGroupLaunch& G) { return md_takes(G, mm8_fits); }
 
-int md_group(int dtype, const MatmulGroupLaunch& G) {
-  if (dtype == kQ8_0 && md_takes_mm8(G)) return launch_mm8(G);
-  if (dtype == kQ4K && md_takes(G, mmk_fits)) return launch_mmk(G);
+// taken: md_takes of G
+int md_group(const MdTune& T, int dtype, const MatmulGroupLaunch& G, bool taken) {
+  if (taken) return dtype == kQ8_0 ? launch_mm8(G) : launch_mmk(G);
   long row_tiles = 0;
   for (int i = 0; i < G.nmat; i++) row_tiles += (G.rows[i] + 31) / 32;
-  const int ks = md_choose(dtype, row_tiles, G.batch, G.bpr);
-  const int nb = md_buffers(dtype, ks, G.batch, G.bpr);
-  if (dtype == kQ8_0) return md_launch<kQ8_0>(G, ks, nb);
-  return dtype == kQ4K ? md_launch<kQ4K>(G, ks, nb) : md_launch<kQ6K>(G, ks, nb);
+  const int ks = md_choose(T, dtype, row_tiles, G.batch, G.bpr);
+  const int nb = md_buffers(T, dtype, ks, G.batch, G.bpr), ex = md_early_x(T, dtype, G.bpr);
+  if (dtype == kQ8_0) return md_launch<kQ8_0>(G, ks, nb, ex);
+  return dtype == kQ4K ? md_launch<kQ4K>(G, ks, nb, ex) : md_launch<kQ6K>(G, ks, nb, ex);
 }
 
 // Register buffers of block loads. K-quants: two (a block's loads issued a
@@ -813,11 +837,9 @@ int md_group(int dtype, const MatmulGroupLaunch& G) {
 // (eight splits of the Qwen3-4B down projection: 30.4 us on one buffer, 34.1
 // on two, which spill). Q8_0: one (on the Llama-3.2-1B shapes at M = 64 one
 // buffer beat two and a ring of four by 4-20%).
-int md_buffers(int dtype, int ks, int batch, int bpr) {
-  const char* nb = getenv("NRQ_MMT_NB");  // tuning override: 1, 2 or 4 (4: Q8_0 only); 8: see md_takes
-  if (nb && nb[0]) return atoi(nb);
-  const char* env = getenv("NRQ_MMT_DB");  // tuning override: 0 (one buffer) or 1 (two)
-  if (env && env[0]) return env[0] == '1' ? 2 : 1;
+int md_buffers(const MdTune& T, int dtype, int ks, int batch, int bpr) {
+  if (T.nb) return atoi(T.nb);
+  if (T.db) return T.db[0] == '1' ? 2 : 1;
   if (dtype == kQ8_0) return 1;
   // whole rows: two buffers, except for rows of fewer than 16 blocks at more
   // than 64 tokens (Qwen3-4B gate and up at M = 512: 58 against 63 us; o's 16
@@ -843,15 +865,15 @@ static MatmulGroupLaunch md_single(const MatmulLaunch& L) {
 // Q8_0 takes the 32 x 32 tiles from 1024 rows (gate/up 8192 x 2048 at M = 64:
 // 25 us against 52 on 16 x 16 tiles; k/v 512 x 2048: 13.6 against 10.6), with
 // 4-byte aligned bases for its dword windows.
-bool mmt_fits(int dtype, const MatmulLaunch& L) {
-  if (dtype == kQ8_0)
-    return (L.rows >= 1024 && (((uintptr_t)L.w | (uintptr_t)L.xs) & 3u) == 0) || md_takes_mm8(md_single(L));
-  return dtype == kQ4K || dtype == kQ6K;
-}
-
+// Below, from 64 tokens, where nrq_mm8.hip takes the matrix.
 int launch_mmt(int dtype, const MatmulLaunch& L) {
-  if (L.rows <= 0 || L.bpr <= 0 || L.batch <= 0) return 0;
-  return md_group(dtype, md_single(L));
+  if (dtype != kQ8_0 && dtype != kQ4K && dtype != kQ6K) return NRQ_LAUNCH_BAD_ARG;
+  const MatmulGroupLaunch G = md_single(L);
+  const bool tiles32 = dtype != kQ8_0 || (L.rows >= 1024 && (((uintptr_t)L.w | (uintptr_t)L.xs) & 3u) == 0);
+  if (!tiles32 && !mm8_fits(G, true)) return NRQ_LAUNCH_BAD_ARG;
+  const MdTune T = md_tune();
+  const bool taken = md_takes(T, dtype, G);
+  return tiles32 || taken ? md_group(T, dtype, G, taken) : NRQ_LAUNCH_BAD_ARG;
 }
 
 // Every matrix of the group in one launch when the 32 x 32 kernel takes their
@@ -867,11 +889,14 @@ int launch_mmt_group(int dtype, const MatmulGroupLaunch& G) {
     bases |= (uintptr_t)G.w[i];
   }
   if (dtype == kQ8_0 && (total < 1024 || (bases & 3u))) return NRQ_LAUNCH_BAD_ARG;
-  if (dtype == kQ8_0 && G.nmat > 1 && !md_takes_mm8(G)) {  // one short matrix does not keep the others from nrq_mm8.hip
+  const MdTune T = md_tune();
+  const bool taken = md_takes(T, dtype, G);
+  if (dtype == kQ8_0 && !taken && G.nmat > 1) {  // one short matrix does not keep the others from nrq_mm8.hip
     for (int i = 0; i < G.nmat; i++)
-      if (md_takes_mm8(md_single({G.w[i], G.xs, G.y[i], G.rows[i], G.bpr, G.batch, G.stream}))) return NRQ_LAUNCH_BAD_ARG;
+      if (md_takes(T, dtype, md_single({G.w[i], G.xs, G.y[i], G.rows[i], G.bpr, G.batch, G.stream})))
+        return NRQ_LAUNCH_BAD_ARG;
   }
-  return md_group(dtype, G);
+  return md_group(T, dtype, G, taken);
 }
 
 // Two groups of different K-quant formats over one activation in one launch,
@@ -888,9 +913,11 @@ int launch_mmt_group2(int dt0, const MatmulGroupLaunch& G0, int dt1, const Matmu
   long row_tiles = 0;
   for (const MatmulGroupLaunch* G : {&G0, &G1})
     for (int i = 0; i < G->nmat; i++) row_tiles += (G->rows[i] + 31) / 32;
-  const int ks = md_choose(dt0, row_tiles, G0.batch, G0.bpr);
-  if (ks < 2 || md_buffers(dt0, ks, G0.batch, G0.bpr) != 1 || md_buffers(dt1, ks, G1.batch, G1.bpr) != 1) return NRQ_LAUNCH_BAD_ARG;
-  return dt0 == kQ4K ? md2_launch_ks<kQ4K, kQ6K>(G0, G1, ks) : md2_launch_ks<kQ6K, kQ4K>(G0, G1, ks);
+  const MdTune T = md_tune();
+  const int ks = md_choose(T, dt0, row_tiles, G0.batch, G0.bpr);
+  if (ks < 2 || md_buffers(T, dt0, ks, G0.batch, G0.bpr) != 1 || md_buffers(T, dt1, ks, G1.batch, G1.bpr) != 1)
+    return NRQ_LAUNCH_BAD_ARG;
+  return dt0 == kQ4K ? md2_launch_ks<kQ4K, kQ6K>(T, G0, G1, ks) : md2_launch_ks<kQ6K, kQ4K>(T, G0, G1, ks);
 }
 
 }  // namespace nrq

@@ -719,6 +719,55 @@ def test_matmul_q4k_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch,
         assert_bitwise(ys[i].cpu().numpy(), want, f"matrix {i} rows {r} bpr {bpr} batch {batch}")
 
 
+def test_matmul_group_reads_the_environment_once(gpu, oracle):
+    """A group of small matrices is bound by the host, so the tuning overrides are read
+    once per launch, not once per variable and matrix: with thousands of other variables
+    in the environment a launch takes at most six lookups' time longer."""
+    import ctypes
+    import os
+    import time
+
+    import torch
+
+    from nightrun_amd import device
+
+    getenv = ctypes.CDLL(None).getenv
+    getenv.argtypes, getenv.restype = [ctypes.c_char_p], ctypes.c_void_p
+    rows, cols, batch = [600, 600, 512], 1024, 8
+    xs = torch.from_numpy(oracle.quantize_act(1, oracle.Rng(7).normal(batch * cols)).view(np.uint8).reshape(-1)).cuda()
+    ws = [torch.from_numpy(np.ascontiguousarray(oracle.gen_weights(1, 8, r, cols)).view(np.uint8).reshape(-1)).cuda()
+          for r in rows]
+    ys = [torch.empty(batch * r, dtype=torch.float32, device="cuda") for r in rows]
+
+    def best(f, n):
+        times = []
+        for _ in range(9):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            for _ in range(n):
+                f()
+            times.append((time.perf_counter() - t) / n)
+        return min(times)
+
+    def launch():
+        device.matmul_group(1, ys, ws, rows, xs, cols, batch)
+
+    def lookup():
+        getenv(b"NRQ_NOT_SET")
+
+    launch()
+    plain, plain_lookup = best(launch, 20), best(lookup, 20)
+    names = [f"PAD_{i}" for i in range(20000)]
+    try:
+        os.environ.update(dict.fromkeys(names, "x"))
+        padded, padded_lookup = best(launch, 20), best(lookup, 20)
+    finally:
+        for name in names:
+            os.environ.pop(name, None)
+    scan = padded_lookup - plain_lookup
+    assert padded - plain < 6 * scan, (plain, padded, scan)
+
+
 @pytest.mark.parametrize("dtype", [1, 2, 3])
 def test_matmul_group(gpu, oracle, dtype):
     """nrq_dev_matmul_group (Acts::matmul_group, infer.rs:180-228): every
