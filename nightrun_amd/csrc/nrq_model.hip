@@ -1500,8 +1500,10 @@ struct nrq_model {
   float *battn = nullptr, *bgate = nullptr, *bup = nullptr, *brope = nullptr;
   uint8_t *bxq = nullptr, *bxq2 = nullptr;
   int* btok = nullptr;
-  float *bqt = nullptr, *batt = nullptr;  // launch_pf_attention's query tiles and weights
+  // launch_pf_attention's query tiles and weights: att_tiles_alloc
+  float *bqt = nullptr, *batt = nullptr;
   size_t batt_bytes = 0;
+  bool att_no_room = false;
   // Sampler (sample.rs:5-21): temperature <= 0 is greedy
   float samp_t = 0.0f, samp_p = 1.0f;
   unsigned long long* rng = nullptr;  // device word, seed | 1
@@ -1849,9 +1851,8 @@ AttGroupCfg att_group(const nrq_model_config& c) {
 // -> 580 at 3000; 64 tokens 376 -> 374 and 804 -> 650; 512 tokens 1312 -> 993
 // and 4632 -> 1827. Qwen3-4B widths, 64 tokens 308 -> 312 and 726 -> 617; 512
 // tokens 1225 -> 987 and 4441 -> 2398. NRQ_ATT_TILES=0 / 1 forces the choice.
-bool att_tiles(const nrq_model* m, int B) {
-  const auto& c = m->cfg;
-  if (!m->batt || (c.head_dim != 64 && c.head_dim != 128)) return false;
+bool att_tiles(const nrq_model_config& c, int B) {
+  if (c.head_dim != 64 && c.head_dim != 128) return false;
   const char* env = getenv("NRQ_ATT_TILES");
   if (env && (env[0] == '0' || env[0] == '1')) return env[0] == '1';
   return (long long)B * c.n_heads >= 2048;
@@ -1862,15 +1863,31 @@ bool att_tiles(const nrq_model* m, int B) {
 // another limit.
 constexpr size_t kPfScratch = (size_t)256 << 20;
 
-int prefill_alloc(nrq_model* m) {
-  if (m->bx) return NRQ_OK;
+// The tiled attention's buffers, before the first chunk that takes it (a model whose
+// head width or chunks never do would hold up to 256 MB unused). Without room for
+// them the other attention kernels take every chunk.
+bool att_tiles_alloc(nrq_model* m) {
+  if (m->batt || m->att_no_room) return !m->att_no_room;
   const auto& c = m->cfg;
-  const size_t B = kMaxBatch, maxd = (size_t)m->maxd;
   // at most a chunk's rows over the whole context; at least one tile per KV head
   const size_t tile = (size_t)c.n_kv_heads * ((c.ctx + 63) & ~63) * nrq::kPfRows * 4;
   const size_t tiles = nrq::pf_tiles(std::min(kMaxBatch, c.ctx), c.n_heads / c.n_kv_heads);
   const char* env = getenv("NRQ_ATT_SCRATCH");
   m->batt_bytes = std::max(tile, std::min(tile * tiles, env ? (size_t)strtoull(env, nullptr, 10) : kPfScratch));
+  const size_t qt = ((size_t)kMaxBatch * m->att_dim + (size_t)c.n_kv_heads * nrq::kPfRows * c.head_dim) * 4;
+  if (hipMalloc((void**)&m->bqt, qt) == hipSuccess && hipMalloc((void**)&m->batt, m->batt_bytes) == hipSuccess)
+    return true;
+  (void)hipGetLastError();
+  if (m->bqt) (void)hipFree(m->bqt);
+  m->bqt = m->batt = nullptr;
+  m->att_no_room = true;
+  return false;
+}
+
+int prefill_alloc(nrq_model* m) {
+  if (m->bx) return NRQ_OK;
+  const auto& c = m->cfg;
+  const size_t B = kMaxBatch, maxd = (size_t)m->maxd;
   struct {
     void** p;
     size_t bytes;
@@ -1881,15 +1898,9 @@ int prefill_alloc(nrq_model* m) {
       {(void**)&m->battn, B * m->att_dim * 4},  {(void**)&m->bgate, B * c.ffn_dim * 4},
       {(void**)&m->bup, B * c.ffn_dim * 4},     {(void**)&m->brope, B * c.head_dim * 4},
       {(void**)&m->bxq, B * act_bytes(NRQ_Q8_0, maxd) + 64}, {(void**)&m->bxq2, B * act_bytes(NRQ_Q4_K, maxd) + 64},
-      {(void**)&m->bqt, (B * m->att_dim + (size_t)c.n_kv_heads * nrq::kPfRows * c.head_dim) * 4},
       {(void**)&m->btok, B * 4},
   };
   for (auto& a : allocs) MHIP(hipMalloc(a.p, a.bytes));
-  // without room for the weights the other attention kernels take every chunk
-  if (hipMalloc((void**)&m->batt, m->batt_bytes) != hipSuccess) {
-    m->batt = nullptr;
-    (void)hipGetLastError();
-  }
   return NRQ_OK;
 }
 
@@ -2001,7 +2012,7 @@ int enqueue_prefill(nrq_model* m, int B) {
   if (hipGetLastError() != hipSuccess) return mfail(NRQ_ERR_DEVICE, "model: embed launch failed");
   const float scale = m->att_scale;
   const float* pending = nullptr;
-  const bool tiles = att_tiles(m, B);
+  const bool tiles = att_tiles(c, B) && att_tiles_alloc(m);
   const int gqa = c.n_heads / c.n_kv_heads;
   int rc;
   for (int l = 0; l < c.n_layers; l++) {

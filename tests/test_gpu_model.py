@@ -578,3 +578,24 @@ def test_prefill_attention_tiles(gpu, oracle, monkeypatch, cfg, n, scratch, fmt)
                 lw["dtypes"][name] = Q4K_M[name]
     prompt = np.random.default_rng(n).integers(0, c["vocab"], n).astype(np.uint32)
     run_pair(oracle, c, w, n + 40, prompt, 3, prefill=True)
+
+
+@pytest.mark.parametrize("cfg,prompts", [(LLAMA_HD96, ((512, False),)), (TINY_GQA4, ((255, False), (256, True)))],
+                         ids=["hd96", "hd64"])
+def test_prefill_attention_tiles_memory(gpu, oracle, cfg, prompts):
+    """The tiled attention's buffers (134 MB at 8192 positions of these widths) are taken
+    by the first chunk of 2048 (token, head) rows and more on 64- or 128-wide heads: not
+    on other head widths, nor by shorter prompts."""
+    import torch
+
+    from nightrun_amd.model import Model
+
+    m = Model(cfg, ctx=8192)
+    m.set_weights(oracle.gen_model(cfg, 4242))
+    free = torch.cuda.mem_get_info()[0]
+    for n, tiles in prompts:
+        m.reset()
+        m.prefill(np.arange(n, dtype=np.uint32) % cfg["vocab"])
+        taken = free - torch.cuda.mem_get_info()[0]
+        assert (taken >= 128 << 20) == tiles and (tiles or taken < 64 << 20), (n, taken)
+    m.close()
