@@ -189,10 +189,13 @@ __device__ __forceinline__ void block_q4(const Q4& L, const uint8_t* st, int lan
 template <int TT>
 __global__ __launch_bounds__(256, 2) void mmk_kernel(MkArgs a) {
   __shared__ __align__(16) uint8_t lds[2 * Stage<TT>::BYTES];
-  // XCD-aware numbering: the token tiles of one row tile share an XCD and its L2
-  const int wg = (int)blockIdx.x, slot = wg >> 3;
-  const int tt = slot % a.ntt, rt = (slot / a.ntt) * 8 + (wg & 7);
-  if (rt >= a.nrt) return;  // padding workgroup
+  // XCD-aware numbering: each XCD takes an eighth of the tiles, those of a row tile
+  // together, which share its L2. Whole row tiles per XCD left some XCDs a third
+  // round of workgroups per CU where the tiles are two rounds (429 tiles, 33 row
+  // tiles x 13: 65 of them on one XCD of 32 CUs)
+  const int idx = ((int)blockIdx.x & 7) * ((int)gridDim.x >> 3) + ((int)blockIdx.x >> 3);
+  if (idx >= a.nrt * a.ntt) return;  // padding workgroup
+  const int rt = idx / a.ntt, tt = idx % a.ntt;
   const int m = rt >= a.tile2 ? 2 : rt >= a.tile1 ? 1 : 0;
   const uint8_t* W = m == 2 ? a.w2 : m == 1 ? a.w1 : a.w0;
   float* Y = m == 2 ? a.y2 : m == 1 ? a.y1 : a.y0;
@@ -300,7 +303,7 @@ int launch_t(const MatmulGroupLaunch& G) {
   a.batch = G.batch;
   a.ntt = (G.batch + Stage<TT>::TOK - 1) / Stage<TT>::TOK;
   a.nrt = n[0] + n[1] + n[2];
-  const long nwg = (long)((a.nrt + 7) / 8) * 8 * a.ntt;
+  const long nwg = ((long)a.nrt * a.ntt + 7) / 8 * 8;
   if (nwg > 0x7fffffffL) return NRQ_LAUNCH_BAD_ARG;
   hipLaunchKernelGGL((mmk_kernel<TT>), dim3((unsigned)nwg), dim3(256), 0, (hipStream_t)G.stream, a);
   return hipGetLastError() == hipSuccess ? NRQ_LAUNCH_OK : NRQ_LAUNCH_FAILED;
@@ -314,15 +317,27 @@ long mmk_tiles(const MatmulGroupLaunch& G, int tok) {
 
 }  // namespace
 
-// Whole tiles (a short one starts early), and enough of them: below about 300
-// workgroups of 128 x 32, or with rows of 32 blocks and more, the splits of
-// nrq_mmt.hip are as fast or faster (2560 x 4096 at 256 tokens, 160 workgroups: 29.7
-// us here, 22.1 there; at 512, 320: 32.7, 33.4; 5120 x 2560 at 256, 320: 21.1, 22.8;
-// 5000 x 3328 at 300, 400: 28.2, 31.0; 2560 x 9728 at 512, 320: 71.6, 71.4).
+// Whole tiles (a short one starts early), and enough of them. The splits of
+// nrq_mmt.hip are as fast or faster (us here, there)
+//  - below 300 workgroups of 128 x 32 (2560 x 4096 at 256 tokens, 160: 29.7, 22.1; from
+//    there 5120 x 2560 at 256, 320: 21.1, 22.8; 2560 x 4096 at 512, 320: 32.7, 33.4;
+//    5000 x 3328 at 300, 400: 28.2, 31.0), and from 18 blocks a row below 450 (7653 x
+//    7680 at 139, 300: 57.7-62.4, 56.9-59.2; from there 4480 x 4864 at 405, 455: 39.9, 43.7);
+//  - with rows of 32 blocks and more (2560 x 9728 at 512, 320: 71.6, 71.4);
+//  - where 128-row tiles make one round of 256 workgroups more than the rows fill, up
+//    to the fourth (2472 + 268 + 7968 x 2048 at 258, 774 for 3024 tiles of 32 x 32:
+//    37.6, 32.3; 3616 + 168 + 4323 x 5632 at 233, 520 for 2040: 58.1, 49.7).
 bool mmk_fits(const MatmulGroupLaunch& G, bool any_size) {
-  for (int i = 0; i < G.nmat; i++)
+  long n32 = 0;
+  for (int i = 0; i < G.nmat; i++) {
     if (G.rows[i] < kRowsWg) return false;
-  return G.batch >= 64 && G.bpr <= (1 << 17) && (any_size || (G.bpr < 32 && mmk_tiles(G, 32) >= 300));
+    n32 += (G.rows[i] + 31) / 32;
+  }
+  if (G.batch < 64 || G.bpr > (1 << 17)) return false;
+  if (any_size) return true;
+  const long tiles = mmk_tiles(G, 32);
+  n32 *= (G.batch + 31) / 32;
+  return G.bpr < 32 && tiles >= (G.bpr < 18 ? 300 : 450) && (tiles > 1024 || (tiles + 255) / 256 <= (n32 + 1023) / 1024);
 }
 
 int launch_mmk(const MatmulGroupLaunch& G) {

@@ -679,7 +679,8 @@ def test_matmul_q8_0_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch
 
 
 @pytest.mark.parametrize("rows_list,bpr,batch,forced", [((128,), 1, 64, True), ((200,), 3, 65, True),
-                                                        ((130, 300, 128), 2, 95, True), ((5000, 4700), 2, 130, False),
+                                                        ((130, 300, 128), 2, 95, True), ((1059, 1035, 2525), 2, 390, True),
+                                                        ((5000, 4700), 2, 130, False),
                                                         ((9000, 8200), 5, 460, False)])
 def test_matmul_q4k_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch, forced):
     """The Q4_K kernel of 64 tokens and more (one or two tiles of 32 tokens per wave): the

@@ -1,0 +1,40 @@
+"""The rules that choose the kernel of a prefill matmul from 64 tokens on: host
+functions of the library, called on shapes alone (no launch, no GPU). Each listed
+shape was measured on the kernel it takes and on the one it would take otherwise."""
+import ctypes as C
+
+import pytest
+
+
+class Group(C.Structure):
+    """MatmulGroupLaunch of nightrun_amd/csrc/nrq_launch.h."""
+    _fields_ = [("w", C.c_void_p * 3), ("y", C.c_void_p * 3), ("rows", C.c_int * 3), ("nmat", C.c_int),
+                ("xs", C.c_void_p), ("bpr", C.c_int), ("batch", C.c_int), ("stream", C.c_void_p)]
+
+
+def group(rows, bpr, batch):
+    g = Group(nmat=len(rows), xs=1 << 20, bpr=bpr, batch=batch)
+    for i, r in enumerate(rows):
+        g.w[i], g.y[i], g.rows[i] = 16 << 20 | i << 30, 17 << 20 | i << 30, r
+    return g
+
+
+def rule(name, *extra):
+    from nightrun_amd import _lib
+
+    fn = getattr(_lib.lib(), name)
+    fn.restype = C.c_bool
+    fn.argtypes = [C.POINTER(Group), *extra]
+    return fn
+
+
+@pytest.mark.parametrize("rows,bpr,batch,takes", [
+    ((9728, 9728), 10, 512, True), ((9728, 9728), 10, 63, False), ((127, 9728), 10, 512, False),
+    ((2560,), 38, 512, False),  # rows of 32 blocks and more
+    ((5120,), 10, 256, True), ((4992,), 10, 224, False),  # 320 workgroups, 273
+    ((3473,), 23, 340, False), ((7653,), 30, 139, False), ((4480,), 19, 405, True),  # 308, 300, 455
+    ((3616, 168, 4323), 22, 233, False), ((2472, 268, 7968), 8, 258, False),  # a round more than the rows fill
+    ((4306,), 27, 403, False), ((6770,), 20, 419, True)])
+def test_q4k_route(rows, bpr, batch, takes):
+    fits = rule("_ZN3nrq8mmk_fitsERKNS_17MatmulGroupLaunchEb", C.c_bool)
+    assert fits(C.byref(group(rows, bpr, batch)), False) == takes
