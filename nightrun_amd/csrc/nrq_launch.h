@@ -106,6 +106,9 @@ int launch_mmt_group(int dtype, const MatmulGroupLaunch& G);
 // the shape and is the faster one (any_size: only the former).
 bool mm8_fits(const MatmulGroupLaunch& G, bool any_size);
 int launch_mm8(const MatmulGroupLaunch& G);
+// A group that matrices of fewer rows than a tile keep from the kernel: whether the
+// others (tall) on it and those in launches of their own are the faster way.
+bool mm8_fits_but_short(const MatmulGroupLaunch& G, MatmulGroupLaunch* tall);
 // Q4_K matrices at 64 tokens and more (nrq_mmk.hip), as for nrq_mm8.hip
 bool mmk_fits(const MatmulGroupLaunch& G, bool any_size);
 int launch_mmk(const MatmulGroupLaunch& G);

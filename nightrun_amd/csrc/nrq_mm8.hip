@@ -358,6 +358,9 @@ static uintptr_t mm8_bases(const MatmulGroupLaunch& G) {
   return b;
 }
 
+// rows start dword aligned
+static bool mm8_even(const MatmulGroupLaunch& G) { return G.bpr % 2 == 0 && (mm8_bases(G) & 3u) == 0; }
+
 bool mm8_fits(const MatmulGroupLaunch& G, bool any_size) {
   long total = 0;
   for (int i = 0; i < G.nmat; i++) {
@@ -368,13 +371,31 @@ bool mm8_fits(const MatmulGroupLaunch& G, bool any_size) {
          (any_size || mm8_tiles(G, Stage<1>::R) >= (total < 1024 ? 48 : 96));
 }
 
+// The short ones' launch takes longer per block than a round here, so two launches pay
+// from 400 workgroups of the others, odd rows 600, and rows of whole stages 280 (6 + 5198
+// x 1472 at 314 tokens, 410: 24.9 us, one launch 42.0; 4822 + 8 x 608 at 404, 532: 25.1,
+// 23.0; 62 + 4121 + 2383 x 1536 at 135, 309: 25.2, 34.6). A group of three in three
+// launches, whatever their sizes: 3000 + 40 + 3200 x 1088 at 67 tokens 30.0, one 16.1.
+bool mm8_fits_but_short(const MatmulGroupLaunch& G, MatmulGroupLaunch* tall) {
+  *tall = G;
+  tall->nmat = 0;
+  for (int i = 0; i < G.nmat; i++) {
+    if (G.rows[i] < Stage<1>::R) continue;
+    tall->w[tall->nmat] = G.w[i];
+    tall->y[tall->nmat] = G.y[i];
+    tall->rows[tall->nmat++] = G.rows[i];
+  }
+  return tall->nmat > 0 && tall->nmat < G.nmat && mm8_fits(*tall, false) &&
+         mm8_tiles(*tall, Stage<1>::R) >= (G.bpr % kS == 0 ? 280 : mm8_even(G) ? 400 : 600);
+}
+
 int launch_mm8(const MatmulGroupLaunch& G) {
   // two tiles per wave where that leaves two workgroups per CU (16384 x 2048 at
   // 512 / 256 / 128 tokens: 73 / 37 / 29 us, one tile 92 / 45 / 25 us)
   bool wide = mm8_tiles(G, Stage<2>::R) >= 512;
   for (int i = 0; i < G.nmat; i++) wide = wide && G.rows[i] >= Stage<2>::R;
   // rows of an odd block count alternate their alignment within a dword
-  if (G.bpr % 2 || (mm8_bases(G) & 3u)) return wide ? launch_t<2, false>(G) : launch_t<1, false>(G);
+  if (!mm8_even(G)) return wide ? launch_t<2, false>(G) : launch_t<1, false>(G);
   return wide ? launch_t<2, true>(G) : launch_t<1, true>(G);
 }
 

@@ -891,10 +891,14 @@ int launch_mmt_group(int dtype, const MatmulGroupLaunch& G) {
   if (dtype == kQ8_0 && (total < 1024 || (bases & 3u))) return NRQ_LAUNCH_BAD_ARG;
   const MdTune T = md_tune();
   const bool taken = md_takes(T, dtype, G);
-  if (dtype == kQ8_0 && !taken && G.nmat > 1) {  // one short matrix does not keep the others from nrq_mm8.hip
-    for (int i = 0; i < G.nmat; i++)
-      if (md_takes(T, dtype, md_single({G.w[i], G.xs, G.y[i], G.rows[i], G.bpr, G.batch, G.stream})))
-        return NRQ_LAUNCH_BAD_ARG;
+  MatmulGroupLaunch tall;
+  if (dtype == kQ8_0 && !taken && !T.nb && !T.splits && !T.db && mm8_fits_but_short(G, &tall)) {
+    int rc = launch_mm8(tall), t = 0;
+    for (int i = 0; i < G.nmat && !rc; i++) {
+      if (t < tall.nmat && G.y[i] == tall.y[t]) t++;
+      else rc = launch_mmq(dtype, {G.w[i], G.xs, G.y[i], G.rows[i], G.bpr, G.batch, G.stream});
+    }
+    return rc;
   }
   return md_group(T, dtype, G, taken);
 }

@@ -637,7 +637,8 @@ def test_matmul_q8_0_spans(gpu, oracle, monkeypatch):
 @pytest.mark.parametrize("rows_list,bpr,batch", [((64,), 8, 64), ((100,), 10, 65), ((6144, 128), 8, 95),
                                                  ((130, 64, 7000), 12, 129), ((8200, 8300), 10, 260),
                                                  ((3000, 40, 3200), 34, 67), ((1531,), 9, 300),
-                                                 ((8200, 8300), 11, 260), ((64,), 31, 64)])
+                                                 ((8200, 8300), 11, 260), ((64,), 31, 64),
+                                                 ((10000, 40, 10100), 24, 130), ((23, 9000, 9100), 11, 160)])
 def test_matmul_q8_0_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch):
     """The Q8_0 kernel of 64 tokens and more (one or two 32 x 32 tiles per wave, stages of
     8 blocks whose last one starts early, as the last row and token tiles do): the smallest

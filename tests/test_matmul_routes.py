@@ -38,3 +38,20 @@ def rule(name, *extra):
 def test_q4k_route(rows, bpr, batch, takes):
     fits = rule("_ZN3nrq8mmk_fitsERKNS_17MatmulGroupLaunchEb", C.c_bool)
     assert fits(C.byref(group(rows, bpr, batch)), False) == takes
+
+
+@pytest.mark.parametrize("rows,bpr,batch,tall", [
+    ((8192, 8192), 64, 512, None), ((545, 758), 67, 224, None), ((1300, 984), 303, 215, None),  # no short one
+    ((3000, 40, 3200), 34, 67, None), ((6, 5198), 46, 314, (5198,)), ((4822, 8), 19, 404, None),
+    ((62, 4121, 2383), 48, 135, (4121, 2383)), ((10000, 40, 10100), 24, 130, (10000, 10100)), ((5, 9), 64, 512, None)])
+def test_q8_0_group_with_short_matrices(rows, bpr, batch, tall):
+    """Groups stay one launch, except that matrices of fewer rows than a tile go alone
+    where the others are large enough; a group without such a matrix never splits."""
+    fits = rule("_ZN3nrq18mm8_fits_but_shortERKNS_17MatmulGroupLaunchEPS0_", C.POINTER(Group))
+    g, h = group(rows, bpr, batch), Group()
+    assert fits(C.byref(g), C.byref(h)) == (tall is not None)
+    if tall:
+        keep = [i for i, r in enumerate(rows) if r in tall]
+        assert tuple(h.rows[:h.nmat]) == tall
+        assert [(h.w[k], h.y[k]) for k in range(h.nmat)] == [(g.w[i], g.y[i]) for i in keep]
+        assert (h.xs, h.bpr, h.batch) == (g.xs, bpr, batch)
