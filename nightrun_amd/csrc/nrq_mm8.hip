@@ -339,13 +339,6 @@ int launch_t(const MatmulGroupLaunch& G) {
 
 }  // namespace
 
-// Whole stages, and whole tiles (a short one starts early). From 96 workgroups of
-// 64 x 64: with fewer, the splits of nrq_mmt.hip keep more of the chip busy (2048 x
-// 2048 at 128 tokens, 64 workgroups: 18.0 us here, 14.4 there; 3072 x 2048 at 128,
-// 96: 17.9 against 25.6; 2048 x 8192 at 256, 128: 63 against 89). Below 1024 rows,
-// where the 16 x 16 tiles of nrq_mmq.hip are the other way, from 48 (512 x 2048 at
-// 512 tokens, 64: 17.8 against 26.0, at 256, 32: 17.8 against 14.4; 600 x 8192 at
-// 300, 50: 62 against 71).
 static long mm8_tiles(const MatmulGroupLaunch& G, int tile) {
   long n = 0;
   for (int i = 0; i < G.nmat; i++) n += (G.rows[i] + tile - 1) / tile;
@@ -361,14 +354,41 @@ static uintptr_t mm8_bases(const MatmulGroupLaunch& G) {
 // rows start dword aligned
 static bool mm8_even(const MatmulGroupLaunch& G) { return G.bpr % 2 == 0 && (mm8_bases(G) & 3u) == 0; }
 
+// Whole stages, and whole tiles (a short one starts early), and enough of them (times:
+// us here, on the kernel that takes the launch otherwise).
+//  - From 96 workgroups of 64 x 64: with fewer, the splits of nrq_mmt.hip keep more of
+//    the chip busy (2048 x 2048 at 128 tokens, 64: 18.0, 14.4; 3072 x 2048 at 128, 96:
+//    17.9, 25.6; 2048 x 8192 at 256, 128: 63, 89). Odd rows, whose two-byte loads cost
+//    more, from where an XCD has more than two of those kernels' tiles per CU (4266 x
+//    1120 at 85, 51 tiles per XCD: 14.1, 13.5; 4643 x 4640 at 84, 57: 41.9, 41.8; 4102 x
+//    736 at 118, 68: 10.1, 11.7; 1191 x 4512 at 395, 65: 39.8, 53.6), and not where the
+//    whole stages are 1.6 times the row (9908 x 288 at 262: 18.8, 15.1).
+//  - Below 1024 rows the other kernel is that of nrq_mmq.hip. Up to two rounds here a
+//    launch takes 0.25 us per block of whole stages and 2.5 or (odd rows) 4 us more; there
+//    0.24 to 0.46 us per block as its workgroups per XCD fill three, four and more rounds of the
+//    CUs, and a fifth more where rows are multiples of 128 bytes (370 x 9856 at 455 tokens, 87 per XCD:
+//    76.7, 69.7; 604 x 6144 at 277, 90: 48.3, 54.8; 674 x 2432 at 305, 120: 22.1, 23.2;
+//    967 x 1600 at 244, 128: 16.5, 15.6; 732 x 1760 at 354, 138: 17.9, 20.5; 517 x 1056
+//    at 456, 145: 13.9, 12.5; 742 x 9824 at 344, 154: 80.8, 106.8).
 bool mm8_fits(const MatmulGroupLaunch& G, bool any_size) {
-  long total = 0;
+  long total = 0, rt32 = 0, rt16 = 0;
   for (int i = 0; i < G.nmat; i++) {
     if (G.rows[i] < Stage<1>::R) return false;
     total += G.rows[i];
+    rt32 += (G.rows[i] + 31) / 32;
+    rt16 += (G.rows[i] + 15) / 16;
   }
-  return G.batch >= kTok && G.bpr >= kS && G.bpr <= (1 << 22) && (mm8_bases(G) & 1u) == 0 &&
-         (any_size || mm8_tiles(G, Stage<1>::R) >= (total < 1024 ? 48 : 96));
+  if (G.batch < kTok || G.bpr < kS || G.bpr > (1 << 22) || (mm8_bases(G) & 1u)) return false;
+  if (any_size) return true;
+  const bool even = mm8_even(G);
+  const long blocks = (long)(G.bpr + kS - 1) / kS * kS;
+  if (total >= 1024)
+    return mm8_tiles(G, Stage<1>::R) >= 96 &&
+           (even || ((rt32 + 7) / 8 * ((G.batch + 31) / 32) > 64 && 10 * blocks < 16L * G.bpr));
+  const long per_xcd = (rt16 + 7) / 8 * ((G.batch + 15) / 16);
+  if (per_xcd > 192) return true;
+  const long there = (per_xcd <= 96 ? 240L : per_xcd <= 128 ? 310L : per_xcd <= 160 ? 380L : 460L) * G.bpr;  // ns
+  return 250 * blocks + (even ? 2500 : 4000) < (G.bpr % 64 ? there : there + there / 5);
 }
 
 // The short ones' launch takes longer per block than a round here, so two launches pay

@@ -55,3 +55,18 @@ def test_q8_0_group_with_short_matrices(rows, bpr, batch, tall):
         assert tuple(h.rows[:h.nmat]) == tall
         assert [(h.w[k], h.y[k]) for k in range(h.nmat)] == [(g.w[i], g.y[i]) for i in keep]
         assert (h.xs, h.bpr, h.batch) == (g.xs, bpr, batch)
+
+
+@pytest.mark.parametrize("rows,bpr,batch,takes", [
+    ((8192, 8192), 64, 512, True), ((8192, 8192), 64, 63, False), ((63, 8192), 64, 512, False),
+    ((3072,), 64, 128, True), ((2048,), 64, 128, False),  # 96 workgroups, 64
+    # odd rows: two tiles of 32 x 32 per CU, and stages of 1.6 times the row
+    ((4266,), 35, 85, False), ((4643,), 145, 84, False), ((4102,), 23, 118, True), ((1191,), 141, 395, True),
+    ((9908,), 9, 262, False),
+    # below 1024 rows
+    ((370,), 308, 455, False), ((604,), 192, 277, True), ((674,), 76, 305, True), ((967,), 50, 244, False),
+    ((732,), 55, 354, True), ((517,), 33, 456, False), ((742,), 307, 344, True), ((709,), 18, 227, False),
+    ((512,), 64, 512, True), ((512,), 64, 256, False), ((600,), 256, 300, True), ((972,), 18, 415, True)])
+def test_q8_0_route(rows, bpr, batch, takes):
+    fits = rule("_ZN3nrq8mm8_fitsERKNS_17MatmulGroupLaunchEb", C.c_bool)
+    assert fits(C.byref(group(rows, bpr, batch)), False) == takes
