@@ -364,12 +364,13 @@ static bool mm8_even(const MatmulGroupLaunch& G) { return G.bpr % 2 == 0 && (mm8
 //    736 at 118, 68: 10.1, 11.7; 1191 x 4512 at 395, 65: 39.8, 53.6), and not where the
 //    whole stages are 1.6 times the row (9908 x 288 at 262: 18.8, 15.1).
 //  - Below 1024 rows the other kernel is that of nrq_mmq.hip. Up to two rounds here a
-//    launch takes 0.25 us per block of whole stages and 2.5 or (odd rows) 4 us more; there
-//    0.24 to 0.46 us per block as its workgroups per XCD fill three, four and more rounds of the
-//    CUs, and a fifth more where rows are multiples of 128 bytes (370 x 9856 at 455 tokens, 87 per XCD:
-//    76.7, 69.7; 604 x 6144 at 277, 90: 48.3, 54.8; 674 x 2432 at 305, 120: 22.1, 23.2;
-//    967 x 1600 at 244, 128: 16.5, 15.6; 732 x 1760 at 354, 138: 17.9, 20.5; 517 x 1056
-//    at 456, 145: 13.9, 12.5; 742 x 9824 at 344, 154: 80.8, 106.8).
+//    launch takes 0.25 us per block of whole stages and 2.5 or (odd rows) 4 us more;
+//    there 0.19 to 0.46 us per block as its workgroups per XCD fill two, three, four and
+//    more rounds of the CUs, and a fifth more where rows are multiples of 128 bytes (225 x
+//    10240 at 371 tokens, 48 per XCD: 82, 63; 370 x 9856 at 455, 87: 76.7, 69.7; 604 x 6144
+//    at 277, 90: 48.3, 54.8; 674 x 2432 at 305, 120: 22.1, 23.2; 967 x 1600 at 244, 128:
+//    16.5, 15.6; 732 x 1760 at 354, 138: 17.9, 20.5; 517 x 1056 at 456, 145: 13.9, 12.5;
+//    742 x 9824 at 344, 154: 80.8, 106.8).
 bool mm8_fits(const MatmulGroupLaunch& G, bool any_size) {
   long total = 0, rt32 = 0, rt16 = 0;
   for (int i = 0; i < G.nmat; i++) {
@@ -381,32 +382,38 @@ bool mm8_fits(const MatmulGroupLaunch& G, bool any_size) {
   if (G.batch < kTok || G.bpr < kS || G.bpr > (1 << 22) || (mm8_bases(G) & 1u)) return false;
   if (any_size) return true;
   const bool even = mm8_even(G);
-  const long blocks = (long)(G.bpr + kS - 1) / kS * kS;
+  const double blocks = (G.bpr + kS - 1) / kS * kS;
   if (total >= 1024)
     return mm8_tiles(G, Stage<1>::R) >= 96 &&
-           (even || ((rt32 + 7) / 8 * ((G.batch + 31) / 32) > 64 && 10 * blocks < 16L * G.bpr));
+           (even || ((rt32 + 7) / 8 * ((G.batch + 31) / 32) > 64 && blocks < 1.6 * G.bpr));
   const long per_xcd = (rt16 + 7) / 8 * ((G.batch + 15) / 16);
   if (per_xcd > 192) return true;
-  const long there = (per_xcd <= 96 ? 240L : per_xcd <= 128 ? 310L : per_xcd <= 160 ? 380L : 460L) * G.bpr;  // ns
-  return 250 * blocks + (even ? 2500 : 4000) < (G.bpr % 64 ? there : there + there / 5);
+  const double there =
+      (per_xcd <= 64 ? 0.19 : per_xcd <= 96 ? 0.24 : per_xcd <= 128 ? 0.31 : per_xcd <= 160 ? 0.38 : 0.46) * G.bpr;
+  return 0.25 * blocks + (even ? 2.5 : 4.0) < (G.bpr % 64 ? there : 1.2 * there);
 }
 
-// The short ones' launch takes longer per block than a round here, so two launches pay
-// from 400 workgroups of the others, odd rows 600, and rows of whole stages 280 (6 + 5198
-// x 1472 at 314 tokens, 410: 24.9 us, one launch 42.0; 4822 + 8 x 608 at 404, 532: 25.1,
-// 23.0; 62 + 4121 + 2383 x 1536 at 135, 309: 25.2, 34.6). A group of three in three
-// launches, whatever their sizes: 3000 + 40 + 3200 x 1088 at 67 tokens 30.0, one 16.1.
+// Two launches cost what the others take here (as above, by rounds of two workgroups
+// per CU) and about 2 us and 0.12 us per block for each short one; one launch of
+// nrq_mmt.hip 3.4 us and 4.2 ns per block and 32 x 32 tile of an XCD. Split where that is
+// 10% more (us split, in one: 6 + 5198 x 1472 at 314 tokens 24.9, 42.0; 9769 + 12 x 8608 at
+// 135: 132, 216; 62 + 4121 + 2383 x 1536 at 135: 25.2, 34.6; 4870 + 41 x 2400 at 188: 33.3, 42.4;
+// 3000 + 40 + 3200 x 1088 at 67: 30.0 in three launches, 16.1).
 bool mm8_fits_but_short(const MatmulGroupLaunch& G, MatmulGroupLaunch* tall) {
   *tall = G;
   tall->nmat = 0;
+  long rt32 = 0;
   for (int i = 0; i < G.nmat; i++) {
+    rt32 += (G.rows[i] + 31) / 32;
     if (G.rows[i] < Stage<1>::R) continue;
     tall->w[tall->nmat] = G.w[i];
     tall->y[tall->nmat] = G.y[i];
     tall->rows[tall->nmat++] = G.rows[i];
   }
-  return tall->nmat > 0 && tall->nmat < G.nmat && mm8_fits(*tall, false) &&
-         mm8_tiles(*tall, Stage<1>::R) >= (G.bpr % kS == 0 ? 280 : mm8_even(G) ? 400 : 600);
+  if (tall->nmat == 0 || tall->nmat == G.nmat || !mm8_fits(*tall, false)) return false;
+  const double blocks = (G.bpr + kS - 1) / kS * kS, rounds = (mm8_tiles(*tall, Stage<1>::R) + 511) / 512;
+  const double split = 0.25 * blocks * rounds + (mm8_even(G) ? 2.5 : 4.0) + (2.0 + 0.12 * G.bpr) * (G.nmat - tall->nmat);
+  return 1.1 * split < 3.4 + 0.0042 * G.bpr * ((rt32 + 7) / 8 * ((G.batch + 31) / 32));
 }
 
 int launch_mm8(const MatmulGroupLaunch& G) {

@@ -42,7 +42,7 @@ def test_q4k_route(rows, bpr, batch, takes):
 
 @pytest.mark.parametrize("rows,bpr,batch,tall", [
     ((8192, 8192), 64, 512, None), ((545, 758), 67, 224, None), ((1300, 984), 303, 215, None),  # no short one
-    ((3000, 40, 3200), 34, 67, None), ((6, 5198), 46, 314, (5198,)), ((4822, 8), 19, 404, None),
+    ((3000, 40, 3200), 34, 67, None), ((6, 5198), 46, 314, (5198,)), ((4870, 41), 75, 188, (4870,)), ((9769, 12), 269, 135, (9769,)),
     ((62, 4121, 2383), 48, 135, (4121, 2383)), ((10000, 40, 10100), 24, 130, (10000, 10100)), ((5, 9), 64, 512, None)])
 def test_q8_0_group_with_short_matrices(rows, bpr, batch, tall):
     """Groups stay one launch, except that matrices of fewer rows than a tile go alone
@@ -64,7 +64,7 @@ def test_q8_0_group_with_short_matrices(rows, bpr, batch, tall):
     ((4266,), 35, 85, False), ((4643,), 145, 84, False), ((4102,), 23, 118, True), ((1191,), 141, 395, True),
     ((9908,), 9, 262, False),
     # below 1024 rows
-    ((370,), 308, 455, False), ((604,), 192, 277, True), ((674,), 76, 305, True), ((967,), 50, 244, False),
+    ((225,), 320, 371, False), ((370,), 308, 455, False), ((604,), 192, 277, True), ((674,), 76, 305, True), ((967,), 50, 244, False),
     ((732,), 55, 354, True), ((517,), 33, 456, False), ((742,), 307, 344, True), ((709,), 18, 227, False),
     ((512,), 64, 512, True), ((512,), 64, 256, False), ((600,), 256, 300, True), ((972,), 18, 415, True)])
 def test_q8_0_route(rows, bpr, batch, takes):
