@@ -48,6 +48,7 @@ struct MkArgs {
   int rows0, rows1, rows2;
   int tile1, tile2;  // first row tile of matrices 1 and 2
   int bpr, batch, ntt, nrt;
+  int whole;  // workgroups per XCD that take whole row tiles
 };
 
 __device__ __forceinline__ i32x16 mfma32(const u32x4& a, const u32x4& b, const i32x16& c) {
@@ -189,13 +190,13 @@ __device__ __forceinline__ void block_q4(const Q4& L, const uint8_t* st, int lan
 template <int TT>
 __global__ __launch_bounds__(256, 2) void mmk_kernel(MkArgs a) {
   __shared__ __align__(16) uint8_t lds[2 * Stage<TT>::BYTES];
-  // XCD-aware numbering: each XCD takes an eighth of the tiles, those of a row tile
-  // together, which share its L2. Whole row tiles per XCD left some XCDs a third
-  // round of workgroups per CU where the tiles are two rounds (429 tiles, 33 row
-  // tiles x 13: 65 of them on one XCD of 32 CUs)
-  const int idx = ((int)blockIdx.x & 7) * ((int)gridDim.x >> 3) + ((int)blockIdx.x >> 3);
-  if (idx >= a.nrt * a.ntt) return;  // padding workgroup
-  const int rt = idx / a.ntt, tt = idx % a.ntt;
+  // XCD-aware numbering: the token tiles of one row tile share an XCD and its L2, eight
+  // neighbouring row tiles at a time; past the first a.whole tiles of each XCD the rest go
+  // round the XCDs one by one
+  const int xcd = (int)blockIdx.x & 7, slot = (int)blockIdx.x >> 3, k = (slot - a.whole) * 8 + xcd;
+  const int rt = slot < a.whole ? slot / a.ntt * 8 + xcd : (a.nrt & ~7) + k / a.ntt;
+  const int tt = slot < a.whole ? slot % a.ntt : k % a.ntt;
+  if (rt >= a.nrt) return;  // padding workgroup
   const int m = rt >= a.tile2 ? 2 : rt >= a.tile1 ? 1 : 0;
   const uint8_t* W = m == 2 ? a.w2 : m == 1 ? a.w1 : a.w0;
   float* Y = m == 2 ? a.y2 : m == 1 ? a.y1 : a.y0;
@@ -303,8 +304,15 @@ int launch_t(const MatmulGroupLaunch& G) {
   a.batch = G.batch;
   a.ntt = (G.batch + Stage<TT>::TOK - 1) / Stage<TT>::TOK;
   a.nrt = n[0] + n[1] + n[2];
-  const long nwg = ((long)a.nrt * a.ntt + 7) / 8 * 8;
-  if (nwg > 0x7fffffffL) return NRQ_LAUNCH_BAD_ARG;
+  // Whole row tiles per XCD, unless the XCDs that take one more than the others then need
+  // a round of workgroups more than the tiles do (4480 x 4864 at 405 tokens, 455 tiles, 35
+  // row tiles x 13: 65 workgroups on three XCDs of 32 CUs: 48.9 us, shared out 41.3). Shared out in every
+  // launch the last nrt % 8 row tiles lose the L2 (5761 x 3840 at 266: 31.5, 33.4).
+  const long all = (long)((a.nrt + 7) / 8) * a.ntt, even = ((long)a.nrt * a.ntt + 7) / 8;
+  const bool share = (all + 31) / 32 > (even + 31) / 32;
+  const long nwg = 8 * (share ? even : all);
+  if (8 * all > 0x7fffffffL) return NRQ_LAUNCH_BAD_ARG;
+  a.whole = (int)(share ? (long)(a.nrt / 8) * a.ntt : all);
   hipLaunchKernelGGL((mmk_kernel<TT>), dim3((unsigned)nwg), dim3(256), 0, (hipStream_t)G.stream, a);
   return hipGetLastError() == hipSuccess ? NRQ_LAUNCH_OK : NRQ_LAUNCH_FAILED;
 }
@@ -321,8 +329,9 @@ long mmk_tiles(const MatmulGroupLaunch& G, int tok) {
 // nrq_mmt.hip are as fast or faster (us here, there)
 //  - below 300 workgroups of 128 x 32 (2560 x 4096 at 256 tokens, 160: 29.7, 22.1; from
 //    there 5120 x 2560 at 256, 320: 21.1, 22.8; 2560 x 4096 at 512, 320: 32.7, 33.4;
-//    5000 x 3328 at 300, 400: 28.2, 31.0), and from 18 blocks a row below 450 (7653 x
-//    7680 at 139, 300: 57.7-62.4, 56.9-59.2; from there 4480 x 4864 at 405, 455: 39.9, 43.7);
+//    5000 x 3328 at 300, 400: 28.2, 31.0), and from 24 blocks a row below 400 (4463 +
+//    6013 x 7936 at 110, 328: 61.1, 59.8; 1798 + 587 + 9648 x 6656 at 97, 384: 52.6, 51.8;
+//    from there 3759 x 7680 at 424, 420: 58.4, 60.8);
 //  - with rows of 32 blocks and more (2560 x 9728 at 512, 320: 71.6, 71.4);
 //  - where 128-row tiles make one round of 256 workgroups more than the rows fill, up
 //    to the fourth (2472 + 268 + 7968 x 2048 at 258, 774 for 3024 tiles of 32 x 32:
@@ -337,7 +346,7 @@ bool mmk_fits(const MatmulGroupLaunch& G, bool any_size) {
   if (any_size) return true;
   const long tiles = mmk_tiles(G, 32);
   n32 *= (G.batch + 31) / 32;
-  return G.bpr < 32 && tiles >= (G.bpr < 18 ? 300 : 450) && (tiles > 1024 || (tiles + 255) / 256 <= (n32 + 1023) / 1024);
+  return G.bpr < 32 && tiles >= (G.bpr < 24 ? 300 : 400) && (tiles > 1024 || (tiles + 255) / 256 <= (n32 + 1023) / 1024);
 }
 
 int launch_mmk(const MatmulGroupLaunch& G) {

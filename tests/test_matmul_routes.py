@@ -32,9 +32,9 @@ def rule(name, *extra):
     ((9728, 9728), 10, 512, True), ((9728, 9728), 10, 63, False), ((127, 9728), 10, 512, False),
     ((2560,), 38, 512, False),  # rows of 32 blocks and more
     ((5120,), 10, 256, True), ((4992,), 10, 224, False),  # 320 workgroups, 273
-    ((3473,), 23, 340, False), ((7653,), 30, 139, False), ((4480,), 19, 405, True),  # 308, 300, 455
+    ((3473,), 23, 340, True), ((4463, 6013), 31, 110, False), ((3759,), 30, 424, True),  # 308, 328, 420
     ((3616, 168, 4323), 22, 233, False), ((2472, 268, 7968), 8, 258, False),  # a round more than the rows fill
-    ((4306,), 27, 403, False), ((6770,), 20, 419, True)])
+    ((4480,), 19, 405, True), ((6770,), 20, 419, True)])
 def test_q4k_route(rows, bpr, batch, takes):
     fits = rule("_ZN3nrq8mmk_fitsERKNS_17MatmulGroupLaunchEb", C.c_bool)
     assert fits(C.byref(group(rows, bpr, batch)), False) == takes
