@@ -728,4 +728,13 @@ __device__ __forceinline__ float dev_expf(float x) {
   return hx > 0x7f800000u ? x : e;
 }
 
+// Where the large kernels of a decode step start: the fused Q8_0 matvecs, 24 KB of code
+// each, the attention and the norm, 22 KB each. A layer runs through about as much code as
+// the instruction cache that two CUs share holds, so the kernels' offsets decide how much
+// of it is still there on the next layer. Llama-3.2-1B widths: gate|up 12.4 to 12.6 us and
+// q|k|v 8.6 on 4 KB boundaries, 13.2 and 9.1 to 9.7 at the offsets that the code before
+// them happened to leave (12.9 and 8.9 at 2 KB, 12.8 and 8.7 at 8 KB), and whole steps
+// moved by up to 2% either way whenever any kernel before them changed its size.
+constexpr int kDecodeEntry = 4096;
+
 }  // namespace nrq

@@ -262,7 +262,7 @@ constexpr int kNormPT = kNormMax / kNormNT;  // values per thread
 // squares together. Workgroup r
 // takes row r of [rows][n] x, add, out, xq and xqk (one row per workgroup in a
 // prefill chunk).
-__global__ __launch_bounds__(kNormNT) void norm_kernel(float* __restrict__ x, const float* __restrict__ add,
+__global__ __attribute__((aligned(kDecodeEntry))) __launch_bounds__(kNormNT) void norm_kernel(float* __restrict__ x, const float* __restrict__ add,
                                                        const float* __restrict__ w, int n, float eps, float rs,
                                                        float* __restrict__ out, uint8_t* __restrict__ xq,
                                                        uint8_t* __restrict__ xqk) {
@@ -460,7 +460,7 @@ constexpr int kAttRing = 3 * 1024 * 16;  // bytes of the value ring: three chunk
 // workgroups of a head share XCD b % 8 and its L2 (needs n_heads % 8 == 0).
 // LDS: att[ctx] | prod[2][kAttProd] | q[hd] | kcur[hd] | vcur[hd] | red[32]
 template <int HD, bool PF = false, int NT = att_threads(HD), int DS = 1>
-__global__ __launch_bounds__(NT) void attention_kernel(
+__global__ __attribute__((aligned(kDecodeEntry))) __launch_bounds__(NT) void attention_kernel(
     const float* __restrict__ q_in, const float* __restrict__ k_in, const float* __restrict__ v_in,
     const float* __restrict__ rope_cs, const int* __restrict__ ctl, int n_heads, int n_kv_heads, int ctx, int layer,
     float scale, uint16_t* __restrict__ kc, uint16_t* __restrict__ vc, float* __restrict__ out,

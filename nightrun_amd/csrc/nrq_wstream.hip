@@ -353,8 +353,14 @@ __device__ __forceinline__ void ws_dma16_g(const void* g, uint32_t m0) {
   asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m0), "v"(g) : "memory");
 }
 
+// The fused Q8_0 kernels start on 4 KB boundaries (kDecodeEntry, nrq_device.h); the others
+// stay as they fall: aligned too, sampled steps of the Qwen3-4B widths take 1% longer.
+__host__ __device__ constexpr int ws_entry(int fmt, int mode) {
+  return fmt == kQ8_0 && (mode & kWsNorm) ? kDecodeEntry : 256;
+}
+
 template <int FMT, int NW, int NS, int MODE>
-__global__ __launch_bounds__(64 * NW) void wstream_matvec(WsArgs A, int bpr, int rpw, int nstages) {
+__global__ __attribute__((aligned(ws_entry(FMT, MODE)))) __launch_bounds__(64 * NW) void wstream_matvec(WsArgs A, int bpr, int rpw, int nstages) {
   constexpr bool NORM = (MODE & kWsNorm) != 0, SWI = (MODE & kWsSwiglu) != 0, URM = (MODE & kWsRowMajorU) != 0;
   constexpr bool QNT = (MODE & kWsQuant) != 0;
   using F = WS<FMT>;

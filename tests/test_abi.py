@@ -44,6 +44,43 @@ def test_library_is_gfx950_only():
         assert other not in blob
 
 
+def _device_functions():
+    """Offset of every device function in its code object, by mangled name."""
+    import struct
+
+    from nightrun_amd import _lib
+
+    blob = open(_lib.LIB_PATH, "rb").read()
+    out = {}
+    for m in re.finditer(b"\x7fELF\x02\x01\x01\x40", blob):  # OS ABI of HSA code objects
+        e = m.start()
+        shoff, = struct.unpack_from("<Q", blob, e + 40)
+        shsize, shnum = struct.unpack_from("<HH", blob, e + 58)
+        sections = [struct.unpack_from("<IIQQQQIIQQ", blob, e + shoff + i * shsize) for i in range(shnum)]
+        for _, kind, _, _, off, size, link, _, _, _ in sections:
+            if kind != 11:  # dynamic symbols
+                continue
+            names = e + sections[link][4]
+            for at in range(e + off, e + off + size, 24):
+                name, info, _, _, value, _ = struct.unpack_from("<IBBHQQ", blob, at)
+                if info & 15 == 2:
+                    out[blob[names + name:blob.index(b"\0", names + name)].decode()] = value
+    return out
+
+
+def test_decode_kernel_entries():
+    """The large kernels of a decode step start on 4 KB boundaries: the fused Q8_0 matvecs
+    (wstream_matvec<1, waves, stages, mode>, odd modes), the attention and the norm. At
+    other offsets, which any change to a kernel before them moves, a step takes up to 3%
+    longer (Llama-3.2-1B widths)."""
+    functions = _device_functions()
+    for pattern, n in ((r"_ZN3nrq14wstream_matvecILi1ELi\d+ELi\d+ELi\d*[13579]E", 4),
+                       (r"_ZN3nrq12_GLOBAL__N_116attention_kernelI", 11), (r"_ZN3nrq12_GLOBAL__N_111norm_kernelE", 1)):
+        entries = {f: v for f, v in functions.items() if re.match(pattern, f)}
+        assert len(entries) == n, pattern
+        assert all(v % 4096 == 0 for v in entries.values()), entries
+
+
 def _no_gpu():
     import torch
 
