@@ -65,6 +65,26 @@ def test_device_expf_sincosf_bitexact(gpu, oracle):
         assert_bitwise(got[~nan], want[~nan], name)
 
 
+def test_device_expf_all_arguments(gpu, oracle):
+    """expf on all 2^32 arguments: its quotient is formed without the IEEE divide."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    import torch
+
+    from nightrun_amd import model
+
+    def differing(hi):
+        bits = np.arange(hi << 24, (hi + 1) << 24, dtype=np.uint32)
+        want = oracle.expf_array(bits.view(np.float32))
+        got = model.mathf(0, torch.from_numpy(bits.view(np.float32)).cuda()).cpu().numpy()
+        bad = got.view(np.uint32) != want.view(np.uint32)
+        bad &= ~(np.isnan(got) & np.isnan(want))
+        return [hex(b) for b in bits[bad][:4]]
+
+    with ThreadPoolExecutor(min(THREADS, 16)) as pool:
+        assert [d for d in pool.map(differing, range(256)) if d] == []
+
+
 def top2_gap(logits):
     """Largest minus second-largest logit: the distance a numeric difference
     would have to move a logit to change the greedy token."""
@@ -578,6 +598,19 @@ def test_prefill_attention_tiles(gpu, oracle, monkeypatch, cfg, n, scratch, fmt)
                 lw["dtypes"][name] = Q4K_M[name]
     prompt = np.random.default_rng(n).integers(0, c["vocab"], n).astype(np.uint32)
     run_pair(oracle, c, w, n + 40, prompt, 3, prefill=True)
+
+
+TILES_WIDE = dict(TINY, n_layers=1, n_heads=32, n_kv_heads=8)
+TILES_LONG = dict(TINY, n_layers=1, vocab=300)
+
+
+@pytest.mark.parametrize("cfg,n", [(TILES_WIDE, 509), (TILES_LONG, 4200)], ids=["groups", "long"])
+def test_prefill_attention_tiles_default(gpu, oracle, cfg, n):
+    """The tiled attention as its rule takes it: 509 four-row tiles of eight KV heads, which
+    the scores kernel takes in groups of two with a single one last; and chunks past
+    position 4096, whose softmax rows pass 64 KB of LDS. Bit-exact."""
+    prompt = np.random.default_rng(n).integers(0, cfg["vocab"], n).astype(np.uint32)
+    run_pair(oracle, cfg, oracle.gen_model(cfg, 960 + n), n + 40, prompt, 3, prefill=True)
 
 
 @pytest.mark.parametrize("cfg,prompts", [(LLAMA_HD96, ((512, False),)), (TINY_GQA4, ((255, False), (256, True)))],

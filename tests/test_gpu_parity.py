@@ -604,8 +604,8 @@ def test_matmul_every_split_count(gpu, oracle, dtype, monkeypatch):
         w = oracle.gen_weights(dtype, 800 + bpr, rows, cols)
         xs = oracle.quantize_act(dtype, oracle.Rng(801 + bpr).normal(batch * cols))
         cases.append((rows, cols, batch, w, xs, oracle.matmul(dtype, 0, w, xs, rows, cols, batch, threads=THREADS)))
-    # register buffers of block loads: 1 or 2, a ring of 4 for Q8_0, and Q8_0's
-    # 8-block spans through LDS (whole rows of 8-block multiples only, else 1)
+    # register buffers of block loads: 1 or 2, a ring of 4 for Q8_0; 8 with one split
+    # names the staged Q8_0 kernel (from 64 tokens and rows of 8 blocks, else one buffer)
     for nb in ("1", "2", "4", "8") if dtype == 1 else ("1", "2"):
         monkeypatch.setenv("NRQ_MMT_NB", nb)
         for ks in ("1", "2", "4", "8"):
@@ -615,10 +615,11 @@ def test_matmul_every_split_count(gpu, oracle, dtype, monkeypatch):
                                f"splits {ks} buffers {nb} rows {rows} cols {cols} batch {batch}")
 
 
-def test_matmul_q8_0_spans(gpu, oracle, monkeypatch):
-    """Q8_0 tiles of whole rows past 64 tokens read 8-block spans of their rows
-    and tokens into LDS: ragged row and token tiles, one span and several, and
-    the span path forced below 64 tokens, all with the oracle's bits."""
+def test_matmul_q8_0_whole_stages(gpu, oracle, monkeypatch):
+    """Q8_0 rows of whole 8-block stages, one stage and several, ragged row and token
+    tiles: as the rules choose (the splits of 32 x 32 tiles at these sizes) and under the
+    override that names the staged kernel, which it takes from 64 tokens; below, that
+    override means one buffer and one split. All with the oracle's bits."""
     cases = []
     for rows, bpr, batch in ((1024, 8, 65), (1100, 16, 130), (1030, 64, 200), (1056, 24, 5), (1024, 8, 33)):
         cols = bpr * 32
@@ -631,25 +632,37 @@ def test_matmul_q8_0_spans(gpu, oracle, monkeypatch):
             monkeypatch.setenv("NRQ_MMT_SPLITS", "1")
         for rows, cols, batch, w, xs, want in cases:
             assert_bitwise(gpu_matmul(1, 0, w, xs, rows, cols, batch), want,
-                           f"spans forced {forced} rows {rows} cols {cols} batch {batch}")
+                           f"forced {forced} rows {rows} cols {cols} batch {batch}")
 
 
-@pytest.mark.parametrize("rows_list,bpr,batch", [((64,), 8, 64), ((100,), 10, 65), ((6144, 128), 8, 95),
-                                                 ((130, 64, 7000), 12, 129), ((8200, 8300), 10, 260),
-                                                 ((3000, 40, 3200), 34, 67), ((1531,), 9, 300),
-                                                 ((8200, 8300), 11, 260), ((64,), 31, 64),
-                                                 ((10000, 40, 10100), 24, 130), ((23, 9000, 9100), 11, 160)])
-def test_matmul_q8_0_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch):
+@pytest.mark.parametrize("rows_list,bpr,batch,way", [((64,), 8, 64, "forced"), ((100,), 10, 65, "forced"),
+                                                     ((6144, 128), 8, 95, "staged"), ((130, 64, 7000), 12, 129, "staged"),
+                                                     ((8200, 8300), 10, 260, "staged"), ((3000, 40, 3200), 34, 67, "other"),
+                                                     ((1531,), 9, 300, "other"), ((1531,), 11, 340, "staged"),
+                                                     ((8200, 8300), 11, 260, "staged"), ((64,), 31, 64, "forced"),
+                                                     ((10000, 40, 10100), 24, 130, "split"),
+                                                     ((23, 9000, 9100), 11, 160, "split")])
+def test_matmul_q8_0_many_tokens(gpu, oracle, monkeypatch, rows_list, bpr, batch, way):
     """The Q8_0 kernel of 64 tokens and more (one or two 32 x 32 tiles per wave, stages of
     8 blocks whose last one starts early, as the last row and token tiles do): the smallest
-    tile, short last tiles and stages, groups with one short matrix, odd block counts
-    (rows two bytes past a dword), and weight scales that are negative, zero, subnormal, the largest f16
-    and, in the last matrix, infinite and NaN, against quants of -128."""
+    tile, short last tiles and stages, groups with one short matrix (in a launch of its own
+    beside large ones, or all in one launch of the 32 x 32 tiles), odd block counts (rows
+    two bytes past a dword), and weight scales that are negative, zero, subnormal, the
+    largest f16 and, in the last matrix, infinite and NaN, against quants of -128."""
+    import ctypes
+
     import torch
 
     from nightrun_amd import device
 
-    if rows_list == (64,):
+    from .test_matmul_routes import Group, group, rule
+
+    g = group(rows_list, bpr, batch)
+    fits = rule("_ZN3nrq8mm8_fitsERKNS_17MatmulGroupLaunchEb", ctypes.c_bool)
+    split = rule("_ZN3nrq18mm8_fits_but_shortERKNS_17MatmulGroupLaunchEPS0_", ctypes.POINTER(Group))
+    assert fits(ctypes.byref(g), way == "forced") == (way in ("forced", "staged"))
+    assert split(ctypes.byref(g), ctypes.byref(Group())) == (way == "split")
+    if way == "forced":
         monkeypatch.setenv("NRQ_MMT_NB", "8")
         monkeypatch.setenv("NRQ_MMT_SPLITS", "1")
     cols = 32 * bpr
