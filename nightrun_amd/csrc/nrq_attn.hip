@@ -17,9 +17,14 @@
 // The weights pass through memory between the launches (the scalar cache does
 // not see vector stores of its own launch).
 // Llama-3.2-1B widths, a 512-token chunk at 1000 positions on average: 51 us
-// scores + 48 us softmax + 64 us values (each product's multiplies and adds
-// alone take 54 us at the VALU rate of one per lane and four clocks), against
-// 650 us for one workgroup per (KV head, token).
+// scores + 48 us softmax + 64 us values, against 650 us for one workgroup per
+// (KV head, token). Each product's multiplies and adds alone take 35 us at the
+// 2.65 clocks in which a SIMD of two waves or more issues an f32 instruction; the
+// rest of a product's time (waits for scalar loads, conversions, launch tails) has
+// not been taken apart. The softmax's LDS (16 bytes per position) leaves fewer workgroups
+// per CU as rows grow, one at 8192 positions: whole prompts of 8000 tokens, two
+// layers, still take a third of the other kernels' time (Llama-3.2-1B widths 33 ms
+// against 88, Qwen3-4B widths 49 against 152).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

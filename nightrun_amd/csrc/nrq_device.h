@@ -694,10 +694,12 @@ __device__ __forceinline__ float wg_chain_nonneg(const float* __restrict__ a, in
 // two-term Remez form, scaled by 2^k (scalbnf: k past f32's exponents in two
 // exact-then-rounded steps). Every range of x runs the same instructions and
 // selects pick its result, so a wave of mixed arguments takes one pass, not
-// the sum of four branches. r*c / (2 - c) has its operands in [2^-27, 1/8] and
-// [1.6, 2.4], so the quotient needs no scaling: a reciprocal, one Newton step
-// and two residual corrections (Markstein) give the rounded value. Equal to
-// the branching form with the IEEE divide on all 2^32 arguments.
+// the sum of four branches. Over all arguments whose quotient r*c / (2 - c) is
+// used, |r*c| is zero or in [2^-58, 0.1271] and 2 - c in [1.67, 2.37], so that
+// neither the quotient nor a residual of 2^-24 of it comes near the subnormals
+// and nothing needs scaling: a reciprocal, one Newton step and two residual
+// corrections (Markstein) give the rounded value. Equal to the branching form
+// with the IEEE divide on all 2^32 arguments (test_device_expf_all_arguments).
 __device__ __forceinline__ float dev_expf(float x) {
   const float ln2hi = 6.9314575195e-01f, ln2lo = 1.4286067653e-06f, invln2 = 1.4426950216e+00f;
   const float P1 = 1.6666625440e-1f, P2 = -2.7667332906e-3f;
@@ -731,10 +733,11 @@ __device__ __forceinline__ float dev_expf(float x) {
 // Where the large kernels of a decode step start: the fused Q8_0 matvecs, 24 KB of code
 // each, the attention and the norm, 22 KB each. A layer runs through about as much code as
 // the instruction cache that two CUs share holds, so the kernels' offsets decide how much
-// of it is still there on the next layer. Llama-3.2-1B widths: gate|up 12.4 to 12.6 us and
-// q|k|v 8.6 on 4 KB boundaries, 13.2 and 9.1 to 9.7 at the offsets that the code before
-// them happened to leave (12.9 and 8.9 at 2 KB, 12.8 and 8.7 at 8 KB), and whole steps
-// moved by up to 2% either way whenever any kernel before them changed its size.
+// of it is still there on the next layer. Llama-3.2-1B widths: gate|up 12.4 to 13.1 us and
+// q|k|v 8.3 to 8.7 on 4 KB boundaries (builds differ in what lies between), 13.2 to 13.4
+// and 9.1 to 9.7 at the offsets that the code before them happened to leave (12.9 and 8.9
+// at 2 KB, 12.8 and 8.7 at 8 KB), and whole steps moved by up to 2% either way whenever any
+// kernel before them changed its size.
 constexpr int kDecodeEntry = 4096;
 
 }  // namespace nrq

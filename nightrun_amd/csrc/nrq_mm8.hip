@@ -5,9 +5,9 @@
 //
 // What bounds it. Per (row, token) and 32-value block the order leaves three
 // roundings that cannot be merged: a multiply by dw, one by dx and the add. At
-// one lane operation per lane and four clocks they cost 192 clocks per 32 x 32
-// tile and block, six times its MFMA step, so everything else is kept off the
-// VALU:
+// the 2.65 clocks in which a SIMD of two waves or more issues an f32 instruction
+// (5.2 with one wave) they cost 127 clocks per 32 x 32 tile and block, four times
+// its MFMA step, so everything else is kept off the VALU:
 //   - f32(acc) costs nothing: the MFMA accumulates onto the bits of 1.5 * 2^23,
 //     so that its result, read as f32, is M = 1.5 * 2^23 + acc (|acc| <= 32 *
 //     128 * 128 < 2^22), and fmaf(M, dw, -(1.5 * 2^23 * dw)) rounds acc * dw once
@@ -26,7 +26,7 @@
 //   - a wave holds RT 32 x 32 tiles of the same 32 tokens, so a token's operands
 //     and d are read once for all of them, and a workgroup of 2 x 2 waves reads
 //     each row and token from memory once.
-// 16384 x 2048 at 512 tokens: 146 -> 68 us (the arithmetic alone takes 41, this
+// 16384 x 2048 at 512 tokens: 146 -> 68 us (the arithmetic alone takes 27, this
 // kernel's steps without their loads 50); 2048 x 8192: 114 -> 64; 3072 x 2048: 37
 // -> 24; 2048 x 2048: 33 -> 19.
 #include "nrq_device.h"

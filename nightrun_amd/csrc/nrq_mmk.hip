@@ -125,7 +125,8 @@ __device__ __forceinline__ void block_q4(const Q4& L, const uint8_t* st, int lan
   for (int j = 0; j < 4; j++) sc0 = sc0 - (float)((scA >> (8 * j)) & 0xffu);
   sc0 = sc0 * ((float)kBias * kUnit);
   // sum_m = sum_k m_{k/2} * bsums[k] (kquant.rs:209-213), bsum = 256 hi + lo, in f16
-  // with f32 sums: all integers below 2^24. Lane half kg holds bsums 8kg .. 8kg+7
+  // with f32 sums: all integers below 2^24 for the bsums of int8 quants (|bsum| <= 16 *
+  // 128; the quantizer writes no others). Lane half kg holds bsums 8kg .. 8kg+7
   const uint32_t mn = kg ? mnB : mnA;
   auto sum_m = [&](int t) {
     u32x4 m, m256;
